@@ -111,6 +111,31 @@ int muzero_dequantize_rows(const uint8_t* packed, int64_t nrows, int64_t packed_
                            int bits, const float* e_table, mz_stream_t stream);
 
 /*
+ * Dequantize a block straight into dense K / V, and copy the unquantized tokens
+ * that follow it.  Replaces: _dequantize_key_range / _dequantize_value_range and
+ * the concatenation with the residual (muzero/cache/layer.py:303-345, :438-459).
+ * packed / mn / scale: the cache's layouts (keys [B, H, tokens/64, D, qb] and
+ * [B, H, tokens/64, D], tokens a multiple of 64; values [B, H, tokens, ng, qb] and
+ * [B, H, tokens, ng], ng = ceil(D/64)), inner dims contiguous, batch / head
+ * strides p_sb, p_sh in bytes, m_sb, m_sh in elements.
+ * out [B, H, tokens + n_tail, D] in out_dtype (o_sb, o_sh, o_st in elements, last
+ * dim contiguous): the values as muzero_dequantize_rows gives them, then
+ * tail [B, H, n_tail, D] of out_dtype (t_sb, t_sh, t_st; may be null if n_tail is 0).
+ */
+typedef struct mz_dequant_args {
+  int batch, heads, tokens, head_dim, bits, n_tail;
+  int meta_dtype, out_dtype;
+  const uint8_t* packed; int64_t p_sb, p_sh;
+  const void* mn; const void* scale; int64_t m_sb, m_sh;
+  const float* e_table;
+  const void* tail; int64_t t_sb, t_sh, t_st;
+  void* out; int64_t o_sb, o_sh, o_st;
+} mz_dequant_args;
+
+int muzero_dequantize_keys(const mz_dequant_args* args, mz_stream_t stream);
+int muzero_dequantize_values(const mz_dequant_args* args, mz_stream_t stream);
+
+/*
  * Logits of one query token per (batch, q-head) against a packed key prefix.
  * Replaces: qk(query, packed_q, mn, scale, output, bits, alpha,
  *   num_key_value_groups, scaling) (muzero/kernels/loader.py:46-49, host

@@ -84,6 +84,20 @@ class AvArgs(ctypes.Structure):
     ]
 
 
+class DequantArgs(ctypes.Structure):
+    """Mirror of ``mz_dequant_args`` (include/muzero_hip.h)."""
+
+    _fields_ = [
+        ("batch", c_int), ("heads", c_int), ("tokens", c_int), ("head_dim", c_int), ("bits", c_int),
+        ("n_tail", c_int), ("meta_dtype", c_int), ("out_dtype", c_int),
+        ("packed", c_vp), ("p_sb", c_i64), ("p_sh", c_i64),
+        ("mn", c_vp), ("scale", c_vp), ("m_sb", c_i64), ("m_sh", c_i64),
+        ("e_table", c_vp),
+        ("tail", c_vp), ("t_sb", c_i64), ("t_sh", c_i64), ("t_st", c_i64),
+        ("out", c_vp), ("o_sb", c_i64), ("o_sh", c_i64), ("o_st", c_i64),
+    ]
+
+
 class PrologueArgs(ctypes.Structure):
     """Mirror of ``mz_prologue_args`` (include/muzero_hip.h)."""
 
@@ -130,6 +144,8 @@ SIGNATURES = {
                                        c_int, c_float, c_vp, c_vp]),
     "muzero_dequantize_rows": (c_int, [c_vp, c_i64, c_i64, c_vp, c_vp, c_int, c_i64, c_vp, c_int, c_i64,
                                        c_int, c_vp, c_vp]),
+    "muzero_dequantize_keys": (c_int, [ctypes.POINTER(DequantArgs), c_vp]),
+    "muzero_dequantize_values": (c_int, [ctypes.POINTER(DequantArgs), c_vp]),
     "muzero_qk": (c_int, [ctypes.POINTER(QkArgs), c_vp]),
     "muzero_av": (c_int, [ctypes.POINTER(AvArgs), c_vp]),
     "muzero_decode_workspace_bytes": (c_i64, [ctypes.POINTER(DecodeArgs), ctypes.POINTER(c_int)]),

@@ -35,9 +35,22 @@ import torch.nn.functional as F
 
 from ..config import MuZeroConfig
 from ..kernels import loader as _k
-from ..quantizer import dequantize_rows, quantize_rows, select_alpha, select_alpha_block
+from ..quantizer import check_codec, dequantize_rows, quantize_rows, select_alpha, select_alpha_block
 
 _STORE_ATTRS = ("packed", "mn", "scale")
+
+
+def _inner_contiguous(t: torch.Tensor) -> torch.Tensor:
+    """``t [B, H, N, K, W]``, copied unless each ``[b, h]`` slice is contiguous (slices of the capacity buffers are)."""
+    k, w = t.shape[3:]
+    return t if t.stride()[2:] == (k * w, w, 1) else t.contiguous()
+
+
+def _has_derivatives(t: torch.Tensor) -> bool:
+    """Whether autograd (reverse or forward mode) or a functorch transform follows ``t``: a kernel's copy
+    of it would drop what they record."""
+    return (type(t) is not torch.Tensor or t.requires_grad or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._functorch.maybe_current_level() is not None)
 
 
 class _PackedStore:
@@ -408,20 +421,18 @@ class MuZeroCacheLayer:
         st.count += t
         return pq, mn, sc
 
-    def _dequantize_span(self, kind: str, start: int, end: int) -> torch.Tensor:
+    def _dequantize_span(self, kind: str, start: int, end: int, tail: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Slots ``[start, end)`` of the kind's packed store as ``[B, H, T, D]`` in the layer
-        dtype.  A key slot is one group of tokens (its rows run along the token axis, one
-        row per channel); a value slot is one token (its rows are the channel groups)."""
+        dtype, followed by ``tail``.  A key slot is one group of tokens (its rows run along the
+        token axis, one row per channel); a value slot is one token (its rows are the channel
+        groups).  The kernels write the dense rows in place (no row tensor, permute or concatenation)."""
         store, d = (self._kstore, self.k_head_dim) if kind == "key" else (self._vstore, self.v_head_dim)
-        tail = self.keys if kind == "key" else self.values
         if store.count == 0 or start >= end:
-            return torch.empty((tail.shape[0], tail.shape[1], 0, d), dtype=self.dtype, device=self.device)
-        packed, mn, scale = (store.view(name, start, end).contiguous() for name in _STORE_ATTRS)
-        rows = self._dequantize_rows(packed.flatten(0, -2), mn.flatten(0, -2), scale.flatten(0, -2), kind)
-        b, h, n = packed.shape[:3]
-        if kind == "key":  # [B, H, groups, D, G] -> tokens along dim 2
-            return rows.reshape(b, h, n, d, self.q_group_size).transpose(3, 4).reshape(b, h, n * self.q_group_size, d)
-        return rows.reshape(b, h, n, -1)[..., :d]
+            window = self.keys if kind == "key" else self.values
+            return torch.empty((window.shape[0], window.shape[1], 0, d), dtype=self.dtype, device=self.device)
+        check_codec(self.amax_eps, self.q_group_size)
+        packed, mn, scale = (_inner_contiguous(store.view(name, start, end)) for name in _STORE_ATTRS)
+        return _k.dequantize_block(packed, mn, scale, kind, self.nbits, float(self._alphas[kind]), d, self.dtype, tail)
 
     def _dequantize_key_range(self, start_group: int, end_group: int) -> torch.Tensor:
         return self._dequantize_span("key", start_group, end_group)
@@ -438,9 +449,15 @@ class MuZeroCacheLayer:
     def dense_kv(self) -> tuple[torch.Tensor, torch.Tensor]:
         """Keys and values of every cached token, ``[B, H, T, D]`` in the layer dtype: the
         packed prefix dequantised, then the residual tail."""
-        k = torch.cat([self._dequantize_key_prefix(), self.keys], dim=2) if self._kstore.count else self.keys
-        v = torch.cat([self._dequantize_value_prefix(), self.values], dim=2) if self._vstore.count else self.values
-        return k, v
+        return self._dense("key"), self._dense("value")
+
+    def _dense(self, kind: str) -> torch.Tensor:
+        store, tail = (self._kstore, self.keys) if kind == "key" else (self._vstore, self.values)
+        if not store.count:
+            return tail
+        if tail.dim() != 4 or _has_derivatives(tail):
+            return torch.cat([self._dequantize_span(kind, 0, store.count), tail], dim=2)
+        return self._dequantize_span(kind, 0, store.count, tail)
 
     # ------------------------------------------------------------------
     # Flush (layer.py:369-396)

@@ -1,4 +1,4 @@
-// Quantize + bit-pack and dequantize kernels (gfx950, wave64).
+// Quantize + bit-pack kernels (gfx950, wave64).
 //
 // Quantize: 2 lanes per 64-value group, 32 consecutive values per lane, so a
 // wave quantizes 32 groups.  The group min/max is an in-lane reduction plus
@@ -719,21 +719,6 @@ __global__ __launch_bounds__(QWG) void quantize_keys_kernel(const void* __restri
   }
 }
 
-// ------------------------------------------------------------- dequantize
-template <int BITS>
-__global__ __launch_bounds__(256) void dequantize_rows_kernel(const uint8_t* __restrict__ packed, int64_t nrows,
-                                                              int64_t ps, const void* mn, const void* sc,
-                                                              int meta_dtype, int64_t ms, void* out, int out_dtype,
-                                                              int64_t os, const float* __restrict__ E) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= nrows) return;
-  constexpr float qmax = (float)((1 << BITS) - 1);
-  const DeqRow r = deq_row(load_any(mn, row * ms, meta_dtype), load_any(sc, row * ms, meta_dtype), qmax, true);
-  const uint32_t q = unpack_code<BITS>(packed + row * ps, lane);
-  store_val(out, row * os + lane, deq_value(r, q, E), out_dtype);
-}
-
 // ------------------------------------------------------------- dispatch
 #define MZ_BITS_SWITCH(BITS, ...)                      \
   switch (BITS) {                                      \
@@ -892,22 +877,6 @@ extern "C" int muzero_quantize_values(const void* values, int x_dtype, int B, in
     if (st2 != MZ_OK) return st2;
   }
   return MZ_OK;
-}
-
-extern "C" int muzero_dequantize_rows(const uint8_t* packed, int64_t nrows, int64_t packed_row_stride,
-                                      const void* mn, const void* scale, int meta_dtype, int64_t meta_stride,
-                                      void* out, int out_dtype, int64_t out_row_stride, int bits,
-                                      const float* e_table, mz_stream_t stream) {
-  if (nrows < 0 || !dtype_ok(meta_dtype) || !dtype_ok(out_dtype) || bits < 1 || bits > 8) return MZ_EINVAL;
-  if (nrows == 0) return MZ_OK;
-  if (!packed || !mn || !scale || !out || !e_table) return MZ_EINVAL;
-  if (packed_row_stride < 8 * bits || out_row_stride < 64 || meta_stride < 1) return MZ_EINVAL;
-  const dim3 grid((unsigned)((nrows + 3) / 4));
-  hipStream_t s = (hipStream_t)stream;
-  MZ_BITS_SWITCH(bits, hipLaunchKernelGGL((dequantize_rows_kernel<B_>), grid, dim3(256), 0, s, packed, nrows,
-                                          packed_row_stride, mn, scale, meta_dtype, meta_stride, out, out_dtype,
-                                          out_row_stride, e_table));
-  return launch_status();
 }
 
 extern "C" const char* muzero_version(void) { return "muzero_hip 0.1.0 gfx950"; }

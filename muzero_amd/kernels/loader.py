@@ -199,6 +199,42 @@ def mu_zero_dequantize_cuda(packed_q: torch.Tensor, mn: torch.Tensor, scale: tor
     check(st, "muzero_dequantize_rows")
 
 
+def dequantize_block(packed: torch.Tensor, mn: torch.Tensor, scale: torch.Tensor, kind: str, bits: int,
+                     alpha: float, head_dim: int, out_dtype: torch.dtype,
+                     tail: torch.Tensor | None = None) -> torch.Tensor:
+    """A packed block as dense ``[B, H, T, D]`` in ``out_dtype``, followed by ``tail [B, H, R, D]`` (same
+    dtype): one launch, no copies.  ``packed / mn / scale`` are views of the cache's key layout
+    (``[B, H, T/64, D, qb]``, ``[B, H, T/64, D, 1]``) or value layout (``[B, H, T, ng, qb]``,
+    ``[B, H, T, ng, 1]``) with contiguous inner dims (reference ``layer.py:303-345``)."""
+    dev = _on_gpu(packed, mn, scale, tail)
+    b, h, n, inner, qb = packed.shape
+    _require(packed.dtype == torch.uint8 and qb == _qbytes(bits) and 1 <= bits <= 8, "packed must be uint8 [..., 8*bits]")
+    _require(inner == (head_dim if kind == "key" else -(-head_dim // GROUP)), "packed block layout")
+    _require(mn.shape == scale.shape == (b, h, n, inner, 1) and mn.dtype == scale.dtype and mn.dtype in DTYPE_ENUM
+             and out_dtype in DTYPE_ENUM, "mn / scale layout and dtypes")
+    _require(packed.stride(4) == 1 and packed.stride(3) == qb and packed.stride(2) == inner * qb, "packed inner layout")
+    _require(mn.stride() == scale.stride() and mn.stride(3) == 1 and mn.stride(2) == inner, "meta inner layout")
+    r = 0 if tail is None else int(tail.shape[2])
+    if r:
+        _require(tail.shape[:2] == (b, h) and tail.shape[3] == head_dim and tail.dtype == out_dtype, "tail layout")
+        if tail.stride(3) != 1:
+            tail = tail.contiguous()
+    tokens = n * GROUP if kind == "key" else n
+    out = torch.empty((b, h, tokens + r, head_dim), dtype=out_dtype, device=dev)
+    a = _lib.DequantArgs()
+    a.batch, a.heads, a.tokens, a.head_dim, a.bits, a.n_tail = b, h, tokens, head_dim, int(bits), r
+    a.meta_dtype, a.out_dtype = DTYPE_ENUM[mn.dtype], DTYPE_ENUM[out_dtype]
+    a.packed, a.p_sb, a.p_sh = ptr(packed), packed.stride(0), packed.stride(1)
+    a.mn, a.scale, a.m_sb, a.m_sh = ptr(mn), ptr(scale), mn.stride(0), mn.stride(1)
+    a.e_table = ptr(tables.device_table("expm1", alpha, dev))
+    if r:
+        a.tail, a.t_sb, a.t_sh, a.t_st = ptr(tail), tail.stride(0), tail.stride(1), tail.stride(2)
+    a.out, a.o_sb, a.o_sh, a.o_st = ptr(out), out.stride(0), out.stride(1), out.stride(2)
+    name = "muzero_dequantize_keys" if kind == "key" else "muzero_dequantize_values"
+    check(getattr(load(), name)(ctypes.byref(a), stream_ptr(dev)), name)
+    return out
+
+
 # --------------------------------------------------------------------------- decode attention
 
 def prepare_mask(attention_mask: torch.Tensor | None, batch: int, length: int) -> torch.Tensor | None:

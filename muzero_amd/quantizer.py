@@ -212,6 +212,13 @@ def _check_group(q_group_size: int) -> None:
         raise MuZeroHipError(f"the HIP kernels implement q_group_size={GROUP}, got {q_group_size}")
 
 
+def check_codec(amax_eps: float, q_group_size: int) -> None:
+    """The dequantize kernels' fixed parameters."""
+    if amax_eps != 1e-8:
+        raise MuZeroHipError("the HIP dequantize kernel implements amax_eps = 1e-8")
+    _check_group(q_group_size)
+
+
 def quantize_rows(
     flat_grouped: torch.Tensor,
     bits: int,
@@ -264,9 +271,7 @@ def dequantize_rows(
     ``mn`` within 1e-8, as in the reference's CUDA kernel (``loader.py:201``);
     the reference's torch expression produces NaN there.
     """
-    if amax_eps != 1e-8:
-        raise MuZeroHipError("the HIP dequantize kernel implements amax_eps = 1e-8")
-    _check_group(q_group_size)
+    check_codec(amax_eps, q_group_size)
     output = torch.empty((packed_q.shape[0], q_group_size), dtype=out_dtype, device=packed_q.device)
     _k.mu_zero_dequantize_cuda(packed_q.contiguous(), mn.contiguous(), scale.contiguous(), output, bits, float(alpha))
     return output
