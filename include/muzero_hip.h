@@ -136,6 +136,28 @@ int muzero_dequantize_keys(const mz_dequant_args* args, mz_stream_t stream);
 int muzero_dequantize_values(const mz_dequant_args* args, mz_stream_t stream);
 
 /*
+ * Alpha statistics of a block x [B, H, T, D] (last dim contiguous), as the cache
+ * flattens it into rows (muzero/quantizer.py:46-55, muzero/cache/layer.py:223-301).
+ * keys != 0: groups of 64 tokens per channel, in order (b, h, t/64, d) (T a multiple
+ * of 64); else groups of 64 channels per token, in order (b, h, t, d/64) (D a
+ * multiple of 64).  offsets[g] = |clamp((0 - min) / max(max - min, 1e-8), 0, 1) - 0.5|
+ * in fp32; sample[i] = |x| in x_dtype at flattened position i * sample_step, i < n_sample.
+ * Rows are read 16 bytes at a time: pointer, strides and D * size multiples of
+ * 16 bytes (offsets too), else MZ_EUNSUPPORTED.
+ */
+int muzero_block_stats(const void* x, int x_dtype, int keys, int B, int H, int T, int D,
+                       int64_t x_sb, int64_t x_sh, int64_t x_st,
+                       float* offsets, void* sample, int64_t n_sample, int64_t sample_step, mz_stream_t stream);
+
+/*
+ * For each of `sets` runs of n non-negative values of `dtype` (run s at values + s * set_stride,
+ * 16-byte aligned): out[s * out_stride + j] = the element of rank kj (0-based) in
+ * ascending order, NaN last (torch.sort's order; the sign bit is ignored).
+ */
+int muzero_select3(const void* values, int dtype, int sets, int64_t set_stride, int64_t n, int64_t k0, int64_t k1,
+                   int64_t k2, float* out, int64_t out_stride, mz_stream_t stream);
+
+/*
  * Logits of one query token per (batch, q-head) against a packed key prefix.
  * Replaces: qk(query, packed_q, mn, scale, output, bits, alpha,
  *   num_key_value_groups, scaling) (muzero/kernels/loader.py:46-49, host

@@ -146,6 +146,9 @@ SIGNATURES = {
                                        c_int, c_vp, c_vp]),
     "muzero_dequantize_keys": (c_int, [ctypes.POINTER(DequantArgs), c_vp]),
     "muzero_dequantize_values": (c_int, [ctypes.POINTER(DequantArgs), c_vp]),
+    "muzero_block_stats": (c_int, [c_vp, c_int, c_int, c_int, c_int, c_int, c_int, c_i64, c_i64, c_i64,
+                                   c_vp, c_vp, c_i64, c_i64, c_vp]),
+    "muzero_select3": (c_int, [c_vp, c_int, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp]),
     "muzero_qk": (c_int, [ctypes.POINTER(QkArgs), c_vp]),
     "muzero_av": (c_int, [ctypes.POINTER(AvArgs), c_vp]),
     "muzero_decode_workspace_bytes": (c_i64, [ctypes.POINTER(DecodeArgs), ctypes.POINTER(c_int)]),

@@ -35,7 +35,7 @@ import torch.nn.functional as F
 
 from ..config import MuZeroConfig
 from ..kernels import loader as _k
-from ..quantizer import check_codec, dequantize_rows, quantize_rows, select_alpha, select_alpha_block
+from ..quantizer import check_codec, dequantize_rows, quantize_rows, select_alpha, select_alpha_block, select_alpha_blocks
 
 _STORE_ATTRS = ("packed", "mn", "scale")
 
@@ -372,6 +372,15 @@ class MuZeroCacheLayer:
                                                         kind=kind, max_points=self.cfg.stats_max_points)
         return alpha
 
+    def _choose_alphas(self, keys: torch.Tensor, values: torch.Tensor) -> None:
+        """Both kinds' alphas from the first blocks flushed, with one wait for their statistics
+        (:meth:`_alpha_for_block` chooses them one at a time where this does not apply)."""
+        if self.nbits != 4 and self._alphas["key"] is None and self._alphas["value"] is None and \
+                self.v_head_dim_padded == values.shape[-1]:
+            self._alphas.update(select_alpha_blocks({"key": keys, "value": values}, bits=self.nbits,
+                                                    q_group_size=self.q_group_size,
+                                                    max_points=self.cfg.stats_max_points))
+
     # ------------------------------------------------------------------
     # Quantise / dequantise
     # ------------------------------------------------------------------
@@ -482,6 +491,8 @@ class MuZeroCacheLayer:
         if not self.is_initialized or self.keys is None or self.values is None:
             return
         k_out, v_out = self._flush_lengths(decode_flush)
+        if k_out and v_out:
+            self._choose_alphas(self.keys[:, :, :k_out], self.values[:, :, :v_out])
         if k_out:
             self._quantize_key_block(self.keys[:, :, :k_out])
             self._kres.drop(k_out)

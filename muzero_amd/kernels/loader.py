@@ -179,6 +179,43 @@ def quantize_value_block_into(values: torch.Tensor, bits: int, alpha: float, eps
     check(st, "muzero_quantize_values")
 
 
+# --------------------------------------------------------------------------- alpha statistics
+
+def stats_block_ok(block: torch.Tensor) -> bool:
+    """Whether :func:`block_statistics` takes ``block [B, H, T, D]``: plain device data whose rows
+    can be read 16 bytes at a time."""
+    es = block.element_size()
+    return (block.is_cuda and type(block) is torch.Tensor and block.dtype in DTYPE_ENUM and block.numel() > 0
+            and block.stride(3) == 1 and block.shape[3] * es % 16 == 0 and block.data_ptr() % 16 == 0
+            and all(s * es % 16 == 0 for s in block.stride()[:3]))
+
+
+def block_statistics(blocks, n_sample: int, step: int, ranks) -> torch.Tensor:
+    """Alpha statistics of ``(block, kind)`` pairs of one size: row i of the result (on the device) holds the
+    elements of the three ranks of the subsample's ``|x|`` (every ``step``-th value of the flattened rows) and
+    the groups' mean zero-anchor offset (reference ``quantizer.py:46-55``).  The mean is torch's, over the
+    offsets in the rows' order."""
+    dev = blocks[0][0].device
+    groups = blocks[0][0].numel() // GROUP
+    pad_g, pad_n = (groups + 3) // 4 * 4, (n_sample + 7) // 8 * 8  # the kernels' 16-byte accesses
+    dtype = blocks[0][0].dtype
+    offsets = torch.empty((len(blocks), pad_g), dtype=torch.float32, device=dev)
+    sample = torch.empty((len(blocks), pad_n), dtype=dtype, device=dev)
+    out = torch.empty((len(blocks), 4), dtype=torch.float32, device=dev)
+    lib, stream = load(), stream_ptr(dev)
+    for i, (block, kind) in enumerate(blocks):
+        b, h, t, d = block.shape
+        check(lib.muzero_block_stats(ptr(block), DTYPE_ENUM[block.dtype], int(kind == "key"), b, h, t, d,
+                                     block.stride(0), block.stride(1), block.stride(2), ptr(offsets[i]),
+                                     ptr(sample[i]), n_sample, step, stream), "muzero_block_stats")
+    check(lib.muzero_select3(ptr(sample), DTYPE_ENUM[dtype], len(blocks), pad_n, n_sample, *ranks, ptr(out), 4, stream),
+          "muzero_select3")
+    for i in range(len(blocks)):
+        # reduced as [1, 1, 1, N], the shape the reference reduces
+        torch.mean(offsets[i, :groups].reshape(1, 1, 1, -1), dim=(0, 1, 2, 3), out=out[i, 3])
+    return out
+
+
 # --------------------------------------------------------------------------- dequantize
 
 def mu_zero_dequantize_cuda(packed_q: torch.Tensor, mn: torch.Tensor, scale: torch.Tensor, output: torch.Tensor,

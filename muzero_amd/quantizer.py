@@ -86,8 +86,40 @@ def select_alpha_block(
     return _decide_alpha(*_block_statistics(block, q_group_size, kind, max_points), bits=bits, kind=kind)
 
 
+def select_alpha_blocks(blocks: dict[str, torch.Tensor], *, bits: int, q_group_size: int,
+                        max_points: int = 65536) -> dict[str, float]:
+    """:func:`select_alpha_block` of one block per kind, with one device round trip for all of them."""
+    if bits != 4 and len({(block.shape, block.dtype) for block in blocks.values()}) == 1 and \
+            all(_kernel_statistics(block, q_group_size, kind, max_points) for kind, block in blocks.items()):
+        stats = _launch_statistics([(block, kind) for kind, block in blocks.items()], max_points)
+        return {kind: _decide_alpha(*row, bits=bits, kind=kind) for kind, row in zip(blocks, stats)}
+    return {kind: select_alpha_block(block, bits=bits, q_group_size=q_group_size, kind=kind, max_points=max_points)
+            for kind, block in blocks.items()}
+
+
+def _kernel_statistics(block: torch.Tensor, q_group_size: int, kind: str, max_points: int) -> bool:
+    """Whether the statistics kernels take the block; others (CPU tensors, odd layouts) run torch operations."""
+    return (q_group_size == GROUP and block.dim() == 4 and block.shape[2 if kind == "key" else 3] % GROUP == 0
+            and 0 < max_points < 1 << 31 and _k.stats_block_ok(block))
+
+
+def _launch_statistics(blocks: list, max_points: int) -> list[list[float]]:
+    """``_alpha_statistics`` of each ``(block, kind)`` (one size) by the statistics kernels."""
+    numel = blocks[0][0].numel()
+    step = 1 if numel <= max_points else max(1, numel // max_points)
+    n = numel if numel <= max_points else min(max_points, -(-numel // step))
+    return _k.block_statistics(blocks, n, step, _percentile_ranks(n)).tolist()
+
+
+def _percentile_ranks(n: int) -> list[int]:
+    """0-based ranks of the 50th, 95th and 99th percentile of n values (``kthvalue``'s k less one)."""
+    return [max(1, int(f * n)) - 1 for f in (0.50, 0.95, 0.99)]
+
+
 def _block_statistics(block: torch.Tensor, q_group_size: int, kind: str, max_points: int) -> list[float]:
     """``_alpha_statistics`` of the rows the cache flattens ``block`` into (see ``select_alpha_block``)."""
+    if _kernel_statistics(block, q_group_size, kind, max_points):
+        return _launch_statistics([(block, kind)], max_points)[0]
     B, H, T, D = (int(x) for x in block.shape)
     G = q_group_size
     dev = block.device
@@ -135,9 +167,8 @@ def _alpha_statistics(sample: torch.Tensor, mn: torch.Tensor, mx: torch.Tensor) 
     """
     eps = 1e-8
     flat = sample.float().abs().reshape(-1)
-    n = flat.numel()
     srt = torch.sort(flat).values
-    ks = [max(1, int(f * n)) - 1 for f in (0.50, 0.95, 0.99)]
+    ks = _percentile_ranks(flat.numel())
     mnf, mxf = mn.float(), mx.float()
     zero_anchor = ((0.0 - mnf) / (mxf - mnf).clamp_min(eps)).clamp(0.0, 1.0)
     anchor_offset = (zero_anchor - 0.5).abs().mean()
