@@ -644,25 +644,79 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // Merge the splits of one (batch, q-head): out = sum_s e^{m_s-M} acc_s / sum_s e^{m_s-M} l_s.
-template <int D>
-__global__ __launch_bounds__(D) void decode_combine_kernel(const float* __restrict__ ws, int n_split, int Hq,
-                                                           void* out, int out_dtype, int64_t out_sb, int64_t out_sh) {
+// Bound by the latency of its loads, so they are all issued before any is
+// waited for: lane s of each wave takes record s's (m, l), and a wave sums the
+// accumulators of records wave, wave + WAVES, ... in runs of COMBINE_LOADS
+// loads (a lane holds D / 64 channels); the waves' sums meet in LDS.  One wave
+// up to 8 splits, four above.  (A loop over the splits that waits for each
+// record cost 0.5 us a split: one sequence of 1000 tokens, 4-bit, 4 / 16 splits
+// 13.2 / 19.0 us per call, now 12.7 / 12.2.)
+constexpr int COMBINE_LOADS = 8;
+template <int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void decode_combine_kernel(const float* __restrict__ ws, int n_split, int Hq,
+                                                                    void* out, int out_dtype, int64_t out_sb,
+                                                                    int64_t out_sh) {
+  constexpr int C = D / 64;  // channels per lane
   const int bh = blockIdx.x;
-  const int c = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float* base = ws + (int64_t)bh * n_split * (D + 2);
-  float M_ = -INFINITY;
-  for (int s = 0; s < n_split; ++s) M_ = fmaxf(M_, base[s * (D + 2) + D]);
-  float num = 0.f, den = 0.f;
+  float num[C], den = 0.f, M_ = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < C; ++k) num[k] = 0.f;
+  // (m, l) of records 64c + lane; past 64 splits the maximum is taken first
+  float m = -INFINITY, l = 0.f;
+  if (lane < n_split) m = base[(int64_t)lane * (D + 2) + D], l = base[(int64_t)lane * (D + 2) + D + 1];
+  float top = m;
+  for (int s = 64 + lane; s < n_split; s += 64) top = fmaxf(top, base[(int64_t)s * (D + 2) + D]);
+  M_ = wave_max_fast(top);
   if (M_ != -INFINITY) {
-    for (int s = 0; s < n_split; ++s) {
-      const float f = __expf(base[s * (D + 2) + D] - M_);
-      num += f * base[s * (D + 2) + c];
-      den += f * base[s * (D + 2) + D + 1];
+    for (int s0 = 0; s0 < n_split; s0 += 64) {
+      if (s0 > 0) {
+        const bool in = s0 + lane < n_split;
+        m = in ? base[(int64_t)(s0 + lane) * (D + 2) + D] : -INFINITY;
+        l = in ? base[(int64_t)(s0 + lane) * (D + 2) + D + 1] : 0.f;
+      }
+      const float f = __expf(m - M_);
+      den += f * l;
+      const int last = min(64, n_split - s0);
+      for (int r0 = wave; r0 < last; r0 += WAVES * COMBINE_LOADS) {
+        float x[COMBINE_LOADS][C];
+#pragma unroll
+        for (int k = 0; k < COMBINE_LOADS; ++k) {
+          // (a record past the last is replaced by the last, with weight 0)
+          const float* rec = base + (int64_t)(s0 + min(r0 + k * WAVES, last - 1)) * (D + 2) + C * lane;
+#pragma unroll
+          for (int c = 0; c < C; ++c) x[k][c] = rec[c];
+        }
+#pragma unroll
+        for (int k = 0; k < COMBINE_LOADS; ++k) {
+          const int r = r0 + k * WAVES;
+          if (r < last) {
+            const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), r));
+#pragma unroll
+            for (int c = 0; c < C; ++c) num[c] += w * x[k][c];
+          }
+        }
+      }
     }
+    den = group_reduce<64>(den, OpAdd());
   }
-  const float o = den > 0.f ? num / den : 0.f;
+  if constexpr (WAVES > 1) {
+    __shared__ float part[WAVES][D];
+#pragma unroll
+    for (int c = 0; c < C; ++c) part[wave][C * lane + c] = num[c];
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w)
+#pragma unroll
+      for (int c = 0; c < C; ++c) num[c] += part[w][C * lane + c];
+  }
   const int b = bh / Hq, h = bh - b * Hq;
-  store_val(out, b * out_sb + (int64_t)h * out_sh + c, o, out_dtype);
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    store_val(out, b * out_sb + (int64_t)h * out_sh + C * lane + c, den > 0.f ? num[c] / den : 0.f, out_dtype);
 }
 
 // The online-softmax state of a packed prefix, for one (batch, q-head): the
@@ -887,8 +941,9 @@ static int launch_combine(const mz_decode_args* a, hipStream_t s) {
   const int64_t need = (int64_t)a->batch * a->kv_heads * a->n_rep * ns * (D + 2) * (int64_t)sizeof(float);
   if (!a->workspace || a->workspace_bytes < need) return MZ_EWORKSPACE;
   const int Hq = a->kv_heads * a->n_rep;
-  hipLaunchKernelGGL((decode_combine_kernel<D>), dim3(a->batch * Hq), dim3(D), 0, s,
-                     (const float*)a->workspace, ns, Hq, a->out, a->out_dtype, a->out_sb, a->out_sh);
+  const auto kernel = ns <= 8 ? decode_combine_kernel<D, 1> : decode_combine_kernel<D, 4>;
+  hipLaunchKernelGGL(kernel, dim3(a->batch * Hq), dim3(ns <= 8 ? 64 : 256), 0, s, (const float*)a->workspace, ns, Hq,
+                     a->out, a->out_dtype, a->out_sb, a->out_sh);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? MZ_OK : (int)e;
 }
