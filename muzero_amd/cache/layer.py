@@ -373,10 +373,9 @@ class MuZeroCacheLayer:
         return alpha
 
     def _choose_alphas(self, keys: torch.Tensor, values: torch.Tensor) -> None:
-        """Both kinds' alphas from the first blocks flushed, with one wait for their statistics
-        (:meth:`_alpha_for_block` chooses them one at a time where this does not apply)."""
-        if self.nbits != 4 and self._alphas["key"] is None and self._alphas["value"] is None and \
-                self.v_head_dim_padded == values.shape[-1]:
+        """Both kinds' alphas (neither set yet) from the first blocks flushed, with one wait for their
+        statistics (:meth:`_alpha_for_block` chooses them one at a time where this does not apply)."""
+        if self.v_head_dim_padded == values.shape[-1]:
             self._alphas.update(select_alpha_blocks({"key": keys, "value": values}, bits=self.nbits,
                                                     q_group_size=self.q_group_size,
                                                     max_points=self.cfg.stats_max_points))
@@ -491,13 +490,15 @@ class MuZeroCacheLayer:
         if not self.is_initialized or self.keys is None or self.values is None:
             return
         k_out, v_out = self._flush_lengths(decode_flush)
-        if k_out and v_out:
-            self._choose_alphas(self.keys[:, :, :k_out], self.values[:, :, :v_out])
+        keys = self.keys[:, :, :k_out] if k_out else None
+        values = self.values[:, :, :v_out] if v_out else None
+        if k_out and v_out and self.nbits != 4 and self._alphas["key"] is None and self._alphas["value"] is None:
+            self._choose_alphas(keys, values)
         if k_out:
-            self._quantize_key_block(self.keys[:, :, :k_out])
+            self._quantize_key_block(keys)
             self._kres.drop(k_out)
         if v_out:
-            self._quantize_value_block(self.values[:, :, :v_out])
+            self._quantize_value_block(values)
             self._vres.drop(v_out)
         self._sync()
 

@@ -780,14 +780,7 @@ static int choose_split(const mz_decode_args* a, int* tiles_per_split) {
   const int n_tiles = a->n_groups + (a->n_residual + kTile - 1) / kTile;
   if (n_tiles <= 0) { *tiles_per_split = 1; return 1; }
   int ns = a->n_split;
-  if (ns <= 0) {
-    // fill the resident workgroup slots (two per CU) once: each workgroup then
-    // loads its tables and query once and runs all its tiles in one pass
-    const int64_t units = std::max<int64_t>(1, (int64_t)a->batch * a->kv_heads);  // an empty batch splits nothing
-    const int64_t slots = 2 * (int64_t)device_cu_count();
-    ns = (int)((slots + units - 1) / units);
-    ns = max(1, min(ns, (n_tiles + 7) / 8));  // at least 2 tiles per wave
-  }
+  if (ns <= 0) ns = choose_splits((int64_t)a->batch * a->kv_heads, n_tiles, kWaves, 2, 0.45f);  // two workgroups per CU
   ns = min(ns, n_tiles);
   const int tps = (n_tiles + ns - 1) / ns;
   *tiles_per_split = tps;
@@ -1072,10 +1065,17 @@ extern "C" int muzero_decode_attention_noalloc(const mz_decode_args* a, mz_strea
     const int c = check_args(a);
     return c != MZ_OK ? c : MZ_EUNSUPPORTED;  // a forced fold path the fold kernel does not take
   }
+  // where the library's own split count does not fit the scratch, fewer splits may
+  if (a->n_split <= 0 && b.batch > 0)
+    while (need > (int64_t)MZ_DECODE_SCRATCH_BYTES && ns > 1) {
+      b.n_split = ns / 2;
+      need = muzero_decode_workspace_bytes(&b, &ns);
+    }
   // the two-pass kernel keeps its logits in the workspace as well: a call
   // whose logits do not fit the scratch runs the general kernel instead
   if (need > (int64_t)MZ_DECODE_SCRATCH_BYTES && b.batch > 0 && which_kernel(&b) == K_TWOPASS) {
     b.kernel_path = MZ_PATH_GENERAL;
+    b.n_split = a->n_split;
     need = muzero_decode_workspace_bytes(&b, &ns);
   }
   // a single split of the other kernels writes the output directly and reads no workspace

@@ -1088,13 +1088,8 @@ bool cb_supported(const mz_decode_args* a) {
 int cb_choose_split(const mz_decode_args* a, int* tiles_per_split) {
   const int n_tiles = a->n_groups + (a->n_residual + cb::TILE - 1) / cb::TILE;
   int ns = a->n_split;
-  if (ns <= 0) {
-    // fill the resident workgroup slots (two per CU) once
-    const int64_t units = std::max<int64_t>(1, (int64_t)a->batch * a->kv_heads);
-    const int64_t slots = 2 * (int64_t)device_cu_count();
-    ns = (int)((slots + units - 1) / units);
-    ns = max(1, min(ns, (n_tiles + 7) / 8));  // at least 2 tiles per wave
-  }
+  // two workgroups per CU; at 1 and 2 bits, more LDS than VALU work, two waves of a SIMD help each other less
+  if (ns <= 0) ns = choose_splits((int64_t)a->batch * a->kv_heads, n_tiles, cb::WAVES, 2, a->bits <= 2 ? 0.7f : 0.45f);
   ns = min(ns, n_tiles);
   const int tps = (n_tiles + ns - 1) / ns;
   *tiles_per_split = tps;

@@ -78,6 +78,51 @@ __device__ __forceinline__ void wave_max2_bound(float& x, float& y) {
   y = __uint_as_float(rb & 0xFFFF0000u);
 }
 
+// The split count of a call the caller leaves to the library (host).  A
+// workgroup of `waves` waves takes one split of a unit's (batch, kv-head)
+// tiles, a tile per wave and round; `per_cu` workgroups are resident per CU.
+// The cost of a count, in rounds of one wave per SIMD (3.2 us for the 4-bit
+// codebook kernel): rounds of the workgroups that run one after another on a
+// slot, a round slowed by `slope` per further wave on the SIMD; 0.05 per wave
+// on the CU; 1.7 per repeated filling of the slots (tables, first loads, a last
+// one that is nearly empty); 0.3 where workgroups share a CU; 0.5 for the merge
+// of the splits.  The counts tried fill the CUs or the slots once, with the
+// fewest splits of the same number of rounds, besides 1 and 2.  Measured
+// (us; a count that fills the slots rounded up, two tiles per wave / this rule):
+// 4-bit, 1 sequence of 1000 tokens 16.3 / 12.3, of 4096 16.9 / 12.7; 48 of 2000
+// 57.2 / 48.0; 70 of 2000 90.1 / 76.1; 7-bit, 1 of 4096 18.2 / 14.5; head_dim 64,
+// 24 of 3001 32.4 / 25.9.
+inline int choose_splits(int64_t units, int n_tiles, int waves, int per_cu, float slope) {
+  units = units < 1 ? 1 : units;  // an empty batch splits nothing
+  const int64_t cus = device_cu_count(), slots = cus * per_cu;
+  auto cost = [&](int ns) {
+    const int tps = (n_tiles + ns - 1) / ns;
+    ns = (n_tiles + tps - 1) / tps;
+    const int64_t wgs = units * ns, fills = (wgs + slots - 1) / slots;
+    const int act = tps < waves ? tps : waves, shared = wgs > cus ? per_cu : 1;
+    const float load = 0.25f * (float)(act * shared);
+    const float round = load > 1.f ? 1.f + slope * (load - 1.f) : 1.f;
+    return (float)fills * ((float)((tps + waves - 1) / waves) * round + 0.05f * (float)(act * shared)) +
+           1.7f * (float)(fills - 1) + (shared > 1 ? 0.3f : 0.f) + (ns > 1 ? 0.5f : 0.f);
+  };
+  int best = 1;
+  float least = cost(1);
+  auto consider = [&](int64_t ns) {
+    if (ns < 2 || ns > n_tiles) return;
+    const float c = cost((int)ns);
+    if (c < least) least = c, best = (int)ns;
+  };
+  consider(2);
+  for (const int64_t cap : {cus, slots}) {
+    const int64_t most = cap / units < n_tiles ? cap / units : n_tiles;
+    if (most < 2) continue;
+    const int64_t tps = (n_tiles + most - 1) / most, rounds = (tps + waves - 1) / waves;
+    consider((n_tiles + rounds * waves - 1) / (rounds * waves));
+    consider(most);
+  }
+  return best;
+}
+
 // Workspace record of one (batch, q-head, split): acc[D], m, l (fp32).
 template <int D>
 __device__ __forceinline__ float* ws_record(const mz_decode_args& a, int b, int qh, int split, int n_split) {

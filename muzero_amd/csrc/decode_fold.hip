@@ -1170,15 +1170,11 @@ int fold_choose_split(const mz_decode_args* a, int* tiles_per_split) {
   const int n_tiles = a->n_groups + (a->n_residual + fold::TILE - 1) / fold::TILE;
   int ns = a->n_split;
   if (ns <= 0) {
-    // fill the resident workgroup slots once: every workgroup then runs its
-    // tiles in one pass with its tables loaded once.  Two workgroups fit a
-    // CU up to 4 query heads per kv-head and 6 bits; the 8-head kernels and
-    // the 7-bit workgroups take a CU alone.
-    const int64_t units = std::max<int64_t>(1, (int64_t)a->batch * a->kv_heads);  // an empty batch splits nothing
+    // two workgroups fit a CU up to 4 query heads per kv-head and 6 bits; the
+    // 8-head kernels and the 7-bit workgroups take a CU alone
     const int per_cu = (a->n_rep > 4 || a->bits >= 7) ? 1 : 2;
-    const int64_t slots = per_cu * (int64_t)device_cu_count();
-    ns = (int)((slots + units - 1) / units);
-    ns = max(1, min(ns, (n_tiles + 7) / 8));  // at least 2 tiles per wave
+    const int waves = a->bits >= 7 && a->n_rep <= 4 ? 8 : 4;
+    ns = choose_splits((int64_t)a->batch * a->kv_heads, n_tiles, waves, per_cu, 0.45f);
   }
   ns = min(ns, n_tiles);
   const int tps = (n_tiles + ns - 1) / ns;

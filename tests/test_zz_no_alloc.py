@@ -70,3 +70,25 @@ def test_noalloc_single_split():
     st, got = _noalloc(plan)
     torch.cuda.synchronize()
     assert st == 0 and torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("hkv,n_rep,length,bits,alpha_v", [(8, 8, 16384, 8, 4.0), (8, 4, 9000, 8, 4.0), (8, 8, 9000, 4, 2.0)])
+def test_noalloc_takes_fewer_splits_where_the_librarys_count_does_not_fit(hkv, n_rep, length, bits, alpha_v):
+    """The split count the library picks with a workspace may need more records than the scratch holds
+    (8 heads, 256 splits, 8 bits: 8.6 MB before the logits); the call then runs with fewer."""
+    from muzero_amd.kernels import loader as L
+    g = torch.Generator(device="cuda").manual_seed(1)
+    lq, d, qb = length // 64 * 64 - 64, 128, 8 * bits
+    q = torch.randn(1, hkv * n_rep, 1, d, generator=g, device="cuda").bfloat16()
+
+    def pack(shape):
+        return (torch.randint(0, 256, (*shape, qb), generator=g, device="cuda", dtype=torch.uint8),
+                -torch.rand(*shape, 1, generator=g, device="cuda").half() - 1, torch.rand(*shape, 1, generator=g, device="cuda").half() + 2)
+    (kp, km, ks), (vp, vm, vs) = pack((1, hkv, lq // 64, d)), pack((1, hkv, lq, 2))
+    res = torch.randn(2, 1, hkv, 64, d, generator=g, device="cuda").bfloat16()
+    plan = L.DecodePlan(q, bits=bits, n_groups=lq // 64, k_packed=kp, k_mn=km, k_scale=ks, v_packed=vp, v_mn=vm, v_scale=vs,
+                        k_res=res[0], v_res=res[1], alpha_key=2.0, alpha_value=alpha_v, scaling=d ** -0.5)
+    want = plan.run().float()
+    st, got = _noalloc(plan)
+    assert st == 0
+    assert (got.float() - want).abs().max().item() < 8e-3  # bf16 outputs below 1: at most an ulp apart
