@@ -266,6 +266,17 @@ typedef struct mz_decode_args {
   int v_prefix;
 } mz_decode_args;
 
+/*
+ * The reference's default decode of one token (muzero/cache/attention.py:179-295) for any head_dim up
+ * to 256, n_rep up to 16 and fp32 queries: muzero_qk over the prefix with the residual's logits, the fp32
+ * softmax, muzero_av with the residual's weighted sum, four launches.  Logits, weights and the prefix's and the
+ * residual's sums are rounded to io_dtype (= out_dtype) where the reference's steps round them.  Reads the
+ * fields of mz_decode_args except the fold tables, n_split, kernel_path and the alphas; packed pointers and strides are multiples of 8 bytes, the workspace is 16-byte
+ * aligned and holds muzero_decode_unfused_workspace_bytes (-1: arguments rejected).
+ */
+int64_t muzero_decode_unfused_workspace_bytes(const mz_decode_args* args);
+int muzero_decode_unfused(const mz_decode_args* args, mz_stream_t stream);
+
 /* Kernel paths of muzero_decode_attention.  Three kernels:
  *  - codebook: attends with the reference's dequantize-then-attend values
  *    (every dequantized value rounded to the layer dtype, bit for bit);

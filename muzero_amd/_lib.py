@@ -159,6 +159,8 @@ SIGNATURES = {
     "muzero_decode_combine": (c_int, [ctypes.POINTER(DecodeArgs), c_vp]),
     "muzero_decode_attention_noalloc": (c_int, [ctypes.POINTER(DecodeArgs), c_vp]),
     "muzero_decode_prefix_state": (c_int, [ctypes.POINTER(DecodeArgs), ctypes.POINTER(PrefixStateArgs), c_vp]),
+    "muzero_decode_unfused_workspace_bytes": (c_i64, [ctypes.POINTER(DecodeArgs)]),
+    "muzero_decode_unfused": (c_int, [ctypes.POINTER(DecodeArgs), c_vp]),
     "muzero_decode_prologue": (c_int, [ctypes.POINTER(PrologueArgs), c_vp]),
     "muzero_stream_read": (c_int, [c_vp, c_i64, c_vp, c_int, c_vp]),
 }

@@ -29,9 +29,9 @@ codebook, two-pass or general kernel), and
 propagates: this build has no dequantize-then-attend fallback to run instead.
 
 Shapes the fused kernels do not take (head_dim other than 64 / 128, fp32
-queries) run the reference's default path itself: the separate ``qk`` / ``av``
-launches (``muzero_qk`` / ``muzero_av``) around a torch softmax and the
-residual matmuls, counted as ``fused_qk_success`` / ``fused_av_success``.
+queries) run the reference's default path itself (``muzero_decode_unfused``:
+qk, softmax, av in four launches, the residual's part in them), counted as
+``fused_qk_success`` / ``fused_av_success``.
 
 Kernel choice, in the reference's environment-switch style (``attention.py:92``,
 ``:110``, ``:128``), ``MUZERO_DECODE_KERNEL``:
@@ -59,6 +59,7 @@ from collections import defaultdict
 import torch
 
 from ..kernels import loader as _k
+from .layer import has_derivatives
 
 _MU_ZERO_DECODE_STATS = defaultdict(int)
 
@@ -188,15 +189,32 @@ def _count_split(key_prefix_length: int, value_prefix_length: int, outcome: str)
 def _split_launches(layer, module, query, attention_mask, scaling, key_prefix_length, value_prefix_length,
                     keys, values, alpha_key, alpha_value):
     """The reference's default decode (``attention.py:179-295``) for shapes the fused kernels
-    do not take (head_dim other than 64 / 128, fp32 queries): ``muzero_qk`` writes the packed
-    prefix's logits in the query dtype, the residual's logits are a torch matmul, the softmax
-    runs in fp32 and is cast to the query dtype, ``muzero_av`` sums the packed values and a
-    torch matmul the residual's.  head_dim up to 256, up to 16 query heads per kv-head."""
-    b, hq, _, d = query.shape
+    do not take (head_dim other than 64 / 128, fp32 queries; head_dim up to 256, up to 16 query heads
+    per kv-head): qk, softmax and av with the residual in them, in four launches.  Calls those do not
+    take (derivatives to record, other layouts) run the steps one by one."""
+    b = query.shape[0]
     n_rep = int(module.num_key_value_groups)
+    length = key_prefix_length + (0 if keys is None else int(keys.shape[2]))
+    mask = _k.prepare_mask(attention_mask, b, length)
+    derivatives = any(t is not None and has_derivatives(t) for t in (query, keys, values, mask))
+    if not derivatives and _k.unfused_decode_ok(query, keys, values, n_rep):
+        return _k.mu_zero_decode_unfused_hip(
+            query, bits=layer.nbits, n_groups=key_prefix_length // layer.q_group_size, value_prefix=value_prefix_length,
+            k_packed=layer._packed_key_q, k_mn=layer._key_mn, k_scale=layer._key_scale,
+            v_packed=layer._packed_value_q, v_mn=layer._value_mn, v_scale=layer._value_scale,
+            k_res=keys, v_res=values, alpha_key=alpha_key, alpha_value=alpha_value, scaling=scaling, mask=mask)
+    return _split_steps(layer, n_rep, query, mask, scaling, key_prefix_length, value_prefix_length, keys, values,
+                        alpha_key, alpha_value)
+
+
+def _split_steps(layer, n_rep, query, mask, scaling, key_prefix_length, value_prefix_length, keys, values,
+                 alpha_key, alpha_value):
+    """The default decode step by step: ``muzero_qk`` writes the packed prefix's logits in the query
+    dtype, the residual's logits are a torch matmul, the softmax runs in fp32 and is cast to the query
+    dtype, ``muzero_av`` sums the packed values and a torch matmul the residual's."""
+    b, hq, _, d = query.shape
     r_k = 0 if keys is None else int(keys.shape[2])
     length = key_prefix_length + r_k
-    mask = _k.prepare_mask(attention_mask, b, length)
     parts = []
     if key_prefix_length > 0:
         logits = torch.empty((b, hq, key_prefix_length), dtype=query.dtype, device=query.device)

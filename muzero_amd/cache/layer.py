@@ -46,7 +46,7 @@ def _inner_contiguous(t: torch.Tensor) -> torch.Tensor:
     return t if t.stride()[2:] == (k * w, w, 1) else t.contiguous()
 
 
-def _has_derivatives(t: torch.Tensor) -> bool:
+def has_derivatives(t: torch.Tensor) -> bool:
     """Whether autograd (reverse or forward mode) or a functorch transform follows ``t``: a kernel's copy
     of it would drop what they record."""
     return (type(t) is not torch.Tensor or t.requires_grad or torch.autograd.forward_ad._current_level >= 0
@@ -463,7 +463,7 @@ class MuZeroCacheLayer:
         store, tail = (self._kstore, self.keys) if kind == "key" else (self._vstore, self.values)
         if not store.count:
             return tail
-        if tail.dim() != 4 or _has_derivatives(tail):
+        if tail.dim() != 4 or has_derivatives(tail):
             return torch.cat([self._dequantize_span(kind, 0, store.count), tail], dim=2)
         return self._dequantize_span(kind, 0, store.count, tail)
 

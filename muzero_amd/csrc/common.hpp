@@ -176,16 +176,6 @@ __device__ __forceinline__ uint32_t pack_byte(uint32_t code, int lane) {
   return acc & 0xFFu;
 }
 
-// Code i (0..63) of a packed row held as bytes in `row` (any alignment).
-template <int BITS>
-__device__ __forceinline__ uint32_t unpack_code(const uint8_t* row, int i) {
-  const int bit = i * BITS;
-  const int byte = bit >> 3;
-  uint32_t w = row[byte];
-  if ((bit & 7) + BITS > 8) w |= (uint32_t)row[byte + 1] << 8;
-  return (w >> (bit & 7)) & ((1u << BITS) - 1u);
-}
-
 // ------------------------------------------------------- dequantization
 // Row parameters recomputed from the STORED metadata (quantizer.py:241-249).
 struct DeqRow {
@@ -219,26 +209,34 @@ __device__ __forceinline__ DeqRow deq_row(float mn, float s, float qmax, bool gu
   return r;
 }
 
-// Exact fp32 dequantized value of code q (quantizer.py:250-255, no FMA).
-__device__ __forceinline__ float deq_value(const DeqRow& r, uint32_t q, const float* E) {
-  const float qf = (float)q;
-  float norm;
-  // d is clamped to the row's 0..bins range so corrupt metadata cannot index
-  // outside the table (for valid metadata the clamp never changes d).
-  if (qf >= r.zl) {
-    const int d = min(max((int)(qf - r.zl), 0), (int)r.pb);
-    const float pn = E[r.offp + d];
-    const float t = r.pe * pn;
-    norm = r.za + t;
-  } else {
-    const int d = min(max((int)(r.zl - qf), 0), (int)r.nb);
-    const float nn = E[r.offn + d];
-    const float t = r.ne * nn;
-    norm = r.za - t;
-  }
-  norm = clamp01(norm);
-  const float u = norm * r.s;
-  return u + r.mn;
+// One group's quantities, the zero level as an integer (0 for NaN metadata,
+// whose values are NaN whatever the table entry) and each side's first table
+// index.
+struct DeqGroup {
+  float mn, s, za, pe, nne;
+  int zl, offp, offn;
+};
+
+template <int QMAX>
+__device__ __forceinline__ DeqGroup make_group(float mn, float s) {
+  const DeqRow r = deq_row(mn, s, (float)QMAX, true);
+  return DeqGroup{r.mn, r.s, r.za, r.pe, -r.ne, r.zl == r.zl ? (int)r.zl : 0, r.offp, r.offn};
+}
+
+// Exact fp32 dequantized value of code q (quantizer.py:250-255, no FMA): the
+// side's table index and coefficient are selected (za - ne*e = za + (-ne)*e);
+// |q - zl| is at most the side's bins.
+// The clamp of the normalised value is v_med3's: it differs from clamp01 only
+// for NaN, which arises from a NaN minimum or from an infinite minimum and
+// scale, and both make the sum below NaN again.
+__device__ __forceinline__ float group_value(const DeqGroup& g, int q, const float* E) {
+  const bool pos = q >= g.zl;
+  const int d = pos ? q - g.zl : g.zl - q;
+  const float e = E[(pos ? g.offp : g.offn) + d];
+  const float t = (pos ? g.pe : g.nne) * e;
+  const float norm = __builtin_amdgcn_fmed3f(g.za + t, 0.f, 1.f);
+  const float u = norm * g.s;
+  return u + g.mn;
 }
 
 }  // namespace mz

@@ -55,35 +55,6 @@ __device__ __forceinline__ void stage_e(float* lds, const float* __restrict__ e,
   __syncthreads();
 }
 
-// One group's quantities, the zero level as an integer (0 for NaN metadata,
-// whose values are NaN whatever the table entry) and each side's first table
-// index.
-struct Group {
-  float mn, s, za, pe, nne;
-  int zl, offp, offn;
-};
-
-template <int BITS>
-__device__ __forceinline__ Group make_group(float mn, float s) {
-  const DeqRow r = deq_row(mn, s, (float)Cfg<BITS>::QMAX, true);
-  return Group{r.mn, r.s, r.za, r.pe, -r.ne, r.zl == r.zl ? (int)r.zl : 0, r.offp, r.offn};
-}
-
-// deq_value without its branch: the side's table index and coefficient are
-// selected (za - ne*e = za + (-ne)*e), |q - zl| is at most the side's bins.
-// The clamp of the normalised value is v_med3's: it differs from clamp01 only
-// for NaN, which arises from a NaN minimum or from an infinite minimum and
-// scale, and both make the sum below NaN again.
-__device__ __forceinline__ float group_value(const Group& g, int q, const float* E) {
-  const bool pos = q >= g.zl;
-  const int d = pos ? q - g.zl : g.zl - q;
-  const float e = E[(pos ? g.offp : g.offn) + d];
-  const float t = (pos ? g.pe : g.nne) * e;
-  const float norm = __builtin_amdgcn_fmed3f(g.za + t, 0.f, 1.f);
-  const float u = norm * g.s;
-  return u + g.mn;
-}
-
 template <int OT>
 __device__ __forceinline__ uint32_t out_bits(float x) {
   if constexpr (OT == MZ_F32) return __float_as_uint(x);
@@ -184,12 +155,12 @@ __global__ __launch_bounds__(Cfg<BITS>::WAVES * 64) void keys_kernel(const Args 
       const uint8_t* rows = a.packed + b * a.psb + h * a.psh + (int64_t)g * a.D * C::QB + t0 * BITS / 8;
       const int64_t m0 = b * a.msb + h * a.msh + (int64_t)g * a.D + c0;
       uint32_t q[W][NW];
-      Group gr[W];
+      DeqGroup gr[W];
 #pragma unroll
       for (int k = 0; k < W; ++k) {
         const int step = k == 0 || two ? k : 0;  // (odd D: the last lane's second channel repeats the first)
         load_bytes<RB>(q[k], rows + (int64_t)(c0 + step) * C::QB);
-        gr[k] = make_group<BITS>(load_any(a.mn, m0 + step, a.mdt), load_any(a.sc, m0 + step, a.mdt));
+        gr[k] = make_group<C::QMAX>(load_any(a.mn, m0 + step, a.mdt), load_any(a.sc, m0 + step, a.mdt));
       }
       if constexpr (C::CB) {
 #pragma unroll
@@ -260,7 +231,7 @@ __global__ __launch_bounds__(Cfg<BITS>::WAVES * 64) void values_kernel(const Arg
     uint32_t q[NW];
     load_bytes<C::QB>(q, a.packed + b * a.psb + h * a.psh + (int64_t)row * a.pst);
     const int64_t m = b * a.msb + h * a.msh + (int64_t)row * a.mst;
-    const Group gr = make_group<BITS>(load_any(a.mn, m, a.mdt), load_any(a.sc, m, a.mdt));
+    const DeqGroup gr = make_group<C::QMAX>(load_any(a.mn, m, a.mdt), load_any(a.sc, m, a.mdt));
     if constexpr (C::CB) {
 #pragma unroll
       for (int v = 0; v <= C::QMAX; ++v) {

@@ -729,3 +729,73 @@ def mu_zero_av_cuda(attn_weights: torch.Tensor, packed_q: torch.Tensor, mn: torc
     a.e_value = ptr(e)
     a.out, a.o_sb, a.o_sh = ptr(output), output.stride(0), output.stride(1)
     check(load().muzero_av(ctypes.byref(a), stream_ptr(dev)), "muzero_av")
+
+
+def unfused_decode_ok(query: torch.Tensor, k_res: torch.Tensor | None, v_res: torch.Tensor | None, n_rep: int) -> bool:
+    """Whether :func:`mu_zero_decode_unfused_hip` takes a decode call of these tensors."""
+    return (query.is_cuda and query.dim() == 4 and query.dtype in DTYPE_ENUM and query.stride(3) == 1
+            and query.shape[3] <= 256 and 1 <= n_rep <= 16 and 0 < query.shape[0] <= 65535
+            and all(t is None or (t.is_cuda and t.device == query.device and t.dtype == query.dtype and t.stride(3) == 1
+                                  and t.shape[:2] == (query.shape[0], query.shape[1] // n_rep)
+                                  and t.shape[3] == query.shape[3]) for t in (k_res, v_res))
+            and query.shape[1] % n_rep == 0)
+
+
+def mu_zero_decode_unfused_hip(query: torch.Tensor, *, bits: int, n_groups: int, value_prefix: int,
+                               k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res,
+                               alpha_key: float, alpha_value: float, scaling: float,
+                               mask: torch.Tensor | None) -> torch.Tensor:
+    """The reference's default decode of one token (``muzero_decode_unfused``): qk with the residual's logits,
+    softmax, av with the residual's weighted sum.  ``query [B, Hq, 1, D]`` (bf16, fp16, fp32), the packed prefix
+    and the residual as :class:`DecodePlan` takes them, ``mask`` additive fp32 ``[B, L]`` or None; returns
+    ``[B, 1, Hq, D]`` in the query dtype (reference ``attention.py:179-295``)."""
+    dev = _on_gpu(query, k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res, mask)
+    b, hq, _, d = query.shape
+    r = 0 if k_res is None else k_res.shape[2]
+    length, qb, ng = GROUP * n_groups + r, _qbytes(bits), (d + GROUP - 1) // GROUP
+    hkv = (k_res if k_res is not None else k_packed).shape[1]
+    a = _lib.DecodeArgs()
+    if n_groups > 0:
+        mn, sc = _meta4(k_mn, "K min"), _meta4(k_scale, "K scale")
+        _require(k_packed.dtype == torch.uint8 and k_packed.shape[:2] == (b, hkv) and k_packed.shape[2] >= n_groups
+                 and tuple(k_packed.shape[3:]) == (d, qb) and k_packed.stride()[2:] == (d * qb, qb, 1), "packed K layout")
+        _require(mn.shape == sc.shape and mn.shape[:2] == (b, hkv) and mn.shape[2] >= n_groups and mn.shape[3] == d
+                 and mn.dtype == sc.dtype and mn.stride() == sc.stride() and mn.stride()[2:] == (d, 1), "K meta layout")
+        a.meta_dtype = DTYPE_ENUM[mn.dtype]
+        a.k_packed, a.kp_sb, a.kp_sh = ptr(k_packed), k_packed.stride(0), k_packed.stride(1)
+        a.k_mn, a.k_scale, a.km_sb, a.km_sh = ptr(mn), ptr(sc), mn.stride(0), mn.stride(1)
+        a.e_key = ptr(tables.device_table("expm1", alpha_key, dev))
+    if value_prefix > 0:
+        mn, sc = _meta4(v_mn, "V min"), _meta4(v_scale, "V scale")
+        _require(v_packed.dtype == torch.uint8 and v_packed.shape[:2] == (b, hkv) and v_packed.shape[2] >= value_prefix
+                 and tuple(v_packed.shape[3:]) == (ng, qb) and v_packed.stride()[2:] == (ng * qb, qb, 1), "packed V layout")
+        _require(mn.shape == sc.shape and mn.shape[:2] == (b, hkv) and mn.shape[2] >= value_prefix and mn.shape[3] == ng
+                 and mn.dtype == sc.dtype and mn.stride() == sc.stride() and mn.stride()[2:] == (ng, 1), "V meta layout")
+        _require(n_groups == 0 or a.meta_dtype == DTYPE_ENUM[mn.dtype], "meta dtypes")
+        a.meta_dtype = DTYPE_ENUM[mn.dtype]
+        a.v_packed, a.vp_sb, a.vp_sh = ptr(v_packed), v_packed.stride(0), v_packed.stride(1)
+        a.v_mn, a.v_scale, a.vm_sb, a.vm_sh = ptr(mn), ptr(sc), mn.stride(0), mn.stride(1)
+        a.e_value = ptr(tables.device_table("expm1", alpha_value, dev))
+    _require(GROUP * n_groups <= value_prefix <= length, "value_prefix must lie between the key prefix and the cache's end")
+    a.v_prefix = value_prefix if value_prefix != GROUP * n_groups else 0
+    if r > 0:
+        n_v = length - value_prefix
+        _require(v_res is not None and v_res.shape[2] >= n_v, "residual K/V lengths differ")
+        a.k_res, a.kr_sb, a.kr_sh, a.kr_st = ptr(k_res), k_res.stride(0), k_res.stride(1), k_res.stride(2)
+        a.v_res, a.vr_sb, a.vr_sh, a.vr_st = ptr(v_res), v_res.stride(0), v_res.stride(1), v_res.stride(2)
+    if mask is not None:
+        a.mask, a.mask_sb = ptr(mask), mask.stride(0)
+    out = torch.empty((b, 1, hq, d), dtype=query.dtype, device=dev)
+    a.batch, a.kv_heads, a.n_rep, a.head_dim, a.bits = b, hkv, hq // hkv, d, int(bits)
+    a.n_groups, a.n_residual = int(n_groups), int(r)
+    a.io_dtype = a.out_dtype = DTYPE_ENUM[query.dtype]
+    a.scaling = float(scaling)
+    a.query, a.q_sb, a.q_sh = ptr(query), query.stride(0), query.stride(1)
+    a.out, a.out_sb, a.out_sh = ptr(out), out.stride(0), out.stride(2)
+    lib, argp = load(), ctypes.byref(a)
+    need = lib.muzero_decode_unfused_workspace_bytes(argp)
+    _require(need >= 0, "unfused decode arguments rejected")
+    workspace = torch.empty(need, dtype=torch.uint8, device=dev)
+    a.workspace, a.workspace_bytes = ptr(workspace), need
+    check(lib.muzero_decode_unfused(argp, stream_ptr(dev)), "muzero_decode_unfused")
+    return out

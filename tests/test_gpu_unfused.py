@@ -1,0 +1,75 @@
+"""The default decode path in four launches (muzero_decode_unfused) against the same path step by step
+(muzero_qk, torch matmuls and softmax, muzero_av): head dims around the kernels' chunks, head counts, types,
+masks, residuals shorter and longer than a workgroup's share, rows longer than the softmax holds in LDS, the
+per-token value flush, and no prefix at all."""
+
+import pytest
+import torch
+
+import muzero_amd as mz
+from muzero_amd.cache import attention as A
+from muzero_amd.cache.layer import MuZeroCacheLayer
+
+pytestmark = pytest.mark.gpu
+BF, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+class _Module:
+    def __init__(self, n_rep):
+        self.num_key_value_groups = n_rep
+
+
+def _both(B, hkv, n_rep, d, tokens, bits, dtype, residual=128, mask=False, logq=False, meta="float16", seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed + d + tokens)
+    k, v = (torch.randn(B, hkv, tokens, d, generator=g, device="cuda").to(dtype) for _ in range(2))
+    q = torch.randn(B, hkv * n_rep, 1, d, generator=g, device="cuda").to(dtype)
+    layer = MuZeroCacheLayer(mz.MuZeroConfig(bits=bits, residual_length=residual, amax_dtype=meta, alpha_key=2.0,
+                                             alpha_value=2.0, logq_compatible_layout=logq))
+    layer.update(k[:, :, :-1], v[:, :, :-1])
+    layer.update(k[:, :, -1:], v[:, :, -1:], {"materialize_full_kv": False})
+    st = layer.get_attention_state()
+    m = None
+    if mask:
+        m = torch.zeros(B, 1, 1, tokens, dtype=dtype, device="cuda")
+        m[0, ..., :tokens // 3] = torch.finfo(dtype).min
+    pre = st["key_prefix_length"], st["value_prefix_length"], layer.keys, layer.values, 2.0, 2.0
+    got = A._split_launches(layer, _Module(n_rep), q, m, d ** -0.5, *pre)
+    prepared = A._k.prepare_mask(m, B, tokens)
+    want = A._split_steps(layer, n_rep, q, prepared, d ** -0.5, *pre)
+    return got, want
+
+
+def _check(got, want):
+    """Logits, weights and the output are rounded at the same places; sums in another order move a few of
+    them to the neighbouring value, so the outputs lie within a few units of the type's rounding."""
+    assert got.shape == want.shape and got.dtype == want.dtype
+    eps = {BF: 2.0 ** -8, F16: 2.0 ** -11, F32: 2.0 ** -19}[got.dtype]
+    rel = (got.double() - want.double()).norm() / want.double().norm()
+    assert rel.item() < 4 * eps, rel.item()
+
+
+@pytest.mark.parametrize("d", [16, 33, 80, 96, 200, 256])
+@pytest.mark.parametrize("n_rep,bits,dtype", [(1, 4, BF), (3, 8, F16), (4, 2, F32), (8, 3, BF), (16, 7, BF)])
+def test_shapes(d, n_rep, bits, dtype):
+    _check(*_both(2, 2, n_rep, d, 777, bits, dtype, mask=n_rep == 3, meta="float32" if dtype == F32 else "bfloat16"))
+
+
+@pytest.mark.parametrize("tokens,residual", [(70, 128), (300, 640), (2100, 320), (14000, 128), (12289, 64)])
+def test_lengths(tokens, residual):
+    _check(*_both(1, 2, 4, 96, tokens, 4, BF, residual=residual, mask=True))
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+def test_values_flushed_per_token(dtype):
+    _check(*_both(2, 2, 4, 96, 500, 4, dtype, residual=64, logq=True))
+
+
+def test_derivatives_run_the_steps():
+    """A query that requires grad keeps the step-by-step path, which differentiates through the residual."""
+    layer = MuZeroCacheLayer(mz.MuZeroConfig(bits=4))
+    k, v = torch.randn(2, 1, 2, 100, 96, device="cuda", dtype=F32)
+    layer.update(k, v)
+    q = torch.randn(1, 4, 1, 96, device="cuda", requires_grad=True)
+    out, _ = mz.mu_zero_decode_attention_forward(_Module(2), q, None, 0.1, layer.get_attention_state())
+    out.sum().backward()
+    assert q.grad is not None and torch.isfinite(q.grad).all()
