@@ -195,8 +195,14 @@ def check(status: int, what: str) -> None:
         raise MuZeroHipError(f"{what} failed with status {status}: {msg}")
 
 
+# the raw handle without a Stream object around it (several us per call), where this torch has the accessor
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(device: torch.device) -> int:
     """Raw hipStream_t of torch's current stream on ``device``."""
+    if _current_raw_stream is not None and device.index is not None:
+        return _current_raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

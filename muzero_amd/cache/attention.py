@@ -109,52 +109,44 @@ def mu_zero_decode_attention_forward(
     if n_groups == 0 and not has_res:
         raise RuntimeError("MuZero attention produced no output; both quantized prefix and dense residual are empty")
 
-    alpha_key = float(layer._selected_alpha_key if layer._selected_alpha_key is not None else 2.0)
-    alpha_value = float(layer._selected_alpha_value if layer._selected_alpha_value is not None else 2.0)
+    alpha_key = layer._selected_alpha_key
+    alpha_value = layer._selected_alpha_value
+    alpha_key = 2.0 if alpha_key is None else float(alpha_key)
+    alpha_value = 2.0 if alpha_value is None else float(alpha_value)
     r = int(keys.shape[2]) if has_res else 0
-    if not _fused_shape(query, module):
-        try:
-            out = _split_launches(layer, module, query, attention_mask, float(scaling), key_prefix_length,
-                                  value_prefix_length, keys if has_res else None, values if has_res else None,
-                                  alpha_key, alpha_value)
-        except Exception:
-            _count_split(key_prefix_length, value_prefix_length, "fallback")
-            raise
-        _count_split(key_prefix_length, value_prefix_length, "success")
-        _MU_ZERO_DECODE_STATS["returns"] += 1
-        return out, None
-    # Decode steps of one layer differ only in the query, the prefix and
-    # residual lengths and the output: once the arguments have been built and
-    # validated for a layer's storage, later steps only patch those fields.
-    fast = getattr(layer, "_hip_decode", None)
-    kernel_path = _kernel_path()
-    key = None
-    if attention_mask is None and has_res and value_prefix_length == key_prefix_length:
-        storage = _storage_key(layer)
-        if storage is not None:
-            key = (storage, query.dtype, tuple(query.shape), query.stride(), layer.nbits, alpha_key,
-                   alpha_value, float(scaling), kernel_path)
+    scaling = float(scaling)
+    fused = _fused_shape(query, module)
+    kernel_path = _kernel_path() if fused else None
     try:
-        out, kernel = _launch(layer, fast, key, query, n_groups, r, has_res, keys, values, alpha_key, alpha_value,
-                              scaling, attention_mask, value_prefix_length, kernel_path)
+        out, kernel = _launch(layer, module, fused, query, attention_mask, n_groups, r, keys if has_res else None,
+                              values if has_res else None, alpha_key, alpha_value, scaling, value_prefix_length,
+                              kernel_path)
     except Exception:
-        _count(key_prefix_length, value_prefix_length, "fallback")
+        (_count if fused else _count_split)(key_prefix_length, value_prefix_length, "fallback")
         raise
-    _count(key_prefix_length, value_prefix_length, "success")
-    _MU_ZERO_DECODE_STATS["hip_fused_decode"] += 1
-    # hip_exact_kernel: calls whose values are the layer-dtype dequantized values (codebook, two-pass, general)
-    _MU_ZERO_DECODE_STATS["hip_fold_kernel" if kernel == "fold" else "hip_exact_kernel"] += 1
-    _MU_ZERO_DECODE_STATS[f"hip_{kernel}_kernel_calls"] += 1
-    _MU_ZERO_DECODE_STATS["returns"] += 1
+    stats = _MU_ZERO_DECODE_STATS
+    if fused:
+        _count(key_prefix_length, value_prefix_length, "success")
+        stats["hip_fused_decode"] += 1
+        # hip_exact_kernel: calls whose values are the layer-dtype dequantized values (codebook, two-pass, general)
+        stats["hip_fold_kernel" if kernel == "fold" else "hip_exact_kernel"] += 1
+        stats[_KERNEL_CALLS[kernel]] += 1
+    else:
+        _count_split(key_prefix_length, value_prefix_length, "success")
+    stats["returns"] += 1
     return out, None
 
 
+_KERNEL_CALLS = {kernel: f"hip_{kernel}_kernel_calls" for kernel in _k.DECODE_KERNELS}
 _KERNEL_PATHS = ("auto", "exact", "fold", "codebook", "general")
 
 
 def _kernel_path() -> str:
     """The decode kernel the environment asks for (``MUZERO_DECODE_KERNEL``)."""
-    path = os.environ.get("MUZERO_DECODE_KERNEL", "auto").strip().lower() or "auto"
+    path = os.environ.get("MUZERO_DECODE_KERNEL")
+    if path is None:
+        return "auto"
+    path = path.strip().lower() or "auto"
     if path not in _KERNEL_PATHS:
         raise ValueError(f"MUZERO_DECODE_KERNEL must be one of {_KERNEL_PATHS}, got {path!r}")
     return path
@@ -184,27 +176,6 @@ def _count_split(key_prefix_length: int, value_prefix_length: int, outcome: str)
         _MU_ZERO_DECODE_STATS[f"fused_qk_{outcome}"] += 1
     if value_prefix_length > 0:
         _MU_ZERO_DECODE_STATS[f"fused_av_{outcome}"] += 1
-
-
-def _split_launches(layer, module, query, attention_mask, scaling, key_prefix_length, value_prefix_length,
-                    keys, values, alpha_key, alpha_value):
-    """The reference's default decode (``attention.py:179-295``) for shapes the fused kernels
-    do not take (head_dim other than 64 / 128, fp32 queries; head_dim up to 256, up to 16 query heads
-    per kv-head): qk, softmax and av with the residual in them, in four launches.  Calls those do not
-    take (derivatives to record, other layouts) run the steps one by one."""
-    b = query.shape[0]
-    n_rep = int(module.num_key_value_groups)
-    length = key_prefix_length + (0 if keys is None else int(keys.shape[2]))
-    mask = _k.prepare_mask(attention_mask, b, length)
-    derivatives = any(t is not None and has_derivatives(t) for t in (query, keys, values, mask))
-    if not derivatives and _k.unfused_decode_ok(query, keys, values, n_rep):
-        return _k.mu_zero_decode_unfused_hip(
-            query, bits=layer.nbits, n_groups=key_prefix_length // layer.q_group_size, value_prefix=value_prefix_length,
-            k_packed=layer._packed_key_q, k_mn=layer._key_mn, k_scale=layer._key_scale,
-            v_packed=layer._packed_value_q, v_mn=layer._value_mn, v_scale=layer._value_scale,
-            k_res=keys, v_res=values, alpha_key=alpha_key, alpha_value=alpha_value, scaling=scaling, mask=mask)
-    return _split_steps(layer, n_rep, query, mask, scaling, key_prefix_length, value_prefix_length, keys, values,
-                        alpha_key, alpha_value)
 
 
 def _split_steps(layer, n_rep, query, mask, scaling, key_prefix_length, value_prefix_length, keys, values,
@@ -259,28 +230,40 @@ def _storage_key(layer):
     return store(ks), store(vs), kr.buf.data_ptr(), kr.start, vr.buf.data_ptr(), vr.start
 
 
-def _launch(layer, fast, key, query, n_groups, r, has_res, keys, values, alpha_key, alpha_value, scaling,
-            attention_mask, value_prefix_length, kernel_path="auto"):
+def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, values, alpha_key, alpha_value, scaling,
+            value_prefix, kernel_path):
+    """One decode call: ``(output, fused kernel or None)``.
+
+    Decode steps of one layer differ only in the query, the mask, the prefix and residual lengths and the
+    output: once the arguments have been built and validated for a layer's storage, later steps only patch
+    those fields (the cached launch is keyed by the storage's addresses, see :func:`_storage_key`)."""
+    key_prefix = n_groups * layer.q_group_size
+    mask = None if attention_mask is None else _k.prepare_mask(attention_mask, query.shape[0], key_prefix + r)
+    n_rep = 0 if fused else int(module.num_key_value_groups)
+    if not fused and (any(t is not None and has_derivatives(t) for t in (query, keys, values, mask))
+                      or not _k.unfused_decode_ok(query, keys, values, n_rep)):
+        return _split_steps(layer, n_rep, query, mask, scaling, key_prefix, value_prefix, keys, values,
+                            alpha_key, alpha_value), None
+    # cached only when every pointer the arguments hold is stable across steps (residual windows in their
+    # decode buffers) and the two prefixes agree
+    key = None
+    if keys is not None and value_prefix == key_prefix:
+        storage = _storage_key(layer)
+        if storage is not None:
+            key = (storage, query.dtype, query.shape, query.stride(), layer.nbits, alpha_key, alpha_value, scaling,
+                   kernel_path, mask is None)
+    fast = getattr(layer, "_hip_decode", None)
     if fast is not None and key is not None and fast.key == key:
-        out = fast.launch(query, n_groups, r)
-        kernel = fast.kernel
+        return fast.launch(query, n_groups, r, mask), fast.kernel
+    prefix = dict(bits=layer.nbits, n_groups=n_groups,
+                  k_packed=layer._packed_key_q, k_mn=layer._key_mn, k_scale=layer._key_scale,
+                  v_packed=layer._packed_value_q, v_mn=layer._value_mn, v_scale=layer._value_scale,
+                  k_res=keys, v_res=values, alpha_key=alpha_key, alpha_value=alpha_value, scaling=scaling,
+                  value_prefix=value_prefix)
+    if fused:
+        plan = _k.DecodePlan(query, attention_mask=mask, kernel_path=kernel_path, **prefix)
     else:
-        plan = _k.DecodePlan(
-            query,
-            bits=layer.nbits,
-            n_groups=n_groups,
-            k_packed=layer._packed_key_q, k_mn=layer._key_mn, k_scale=layer._key_scale,
-            v_packed=layer._packed_value_q, v_mn=layer._value_mn, v_scale=layer._value_scale,
-            k_res=keys if has_res else None, v_res=values if has_res else None,
-            alpha_key=alpha_key, alpha_value=alpha_value,
-            scaling=float(scaling),
-            attention_mask=attention_mask,
-            value_prefix=value_prefix_length,
-            kernel_path=kernel_path,
-        )
-        out = plan.run()
-        kernel = plan.kernel
-        # cache the validated arguments only when every pointer they hold is
-        # stable across steps (residual windows in their decode buffers, no mask)
-        layer._hip_decode = _k.StepDecode(plan, key) if key is not None else None
-    return out, kernel
+        plan = _k.UnfusedPlan(query, mask=mask, **prefix)
+    out = plan.run()
+    layer._hip_decode = _k.StepDecode(plan, key) if key is not None else None
+    return out, plan.kernel

@@ -124,7 +124,7 @@ class _ResidualWindow:
 
     def _refresh(self) -> None:
         # the tokens as one tensor, made once per change (the decode path reads it often)
-        self.view = self.buf[:, :, self.start:self.end] if self.buf is not None else self.loose
+        self.view = self.loose if self.buf is None else self.buf.narrow(2, self.start, self.end - self.start)
 
     def tokens(self) -> Optional[torch.Tensor]:
         return self.view
@@ -138,10 +138,10 @@ class _ResidualWindow:
         self.loose = self.view = t
 
     def _room_for_one(self, min_cap: int) -> None:
+        if self.buf is not None and self.end < self.buf.shape[2]:
+            return
         live = self.tokens()
         n = len(self)
-        if self.buf is not None and self.end < int(self.buf.shape[2]):
-            return
         cap = max(min_cap, n + 1)
         cap = -(-cap // self.align) * self.align
         buf = torch.empty((*live.shape[:2], cap, live.shape[3]), dtype=live.dtype, device=live.device)
@@ -153,7 +153,7 @@ class _ResidualWindow:
     def slot(self, min_cap: int) -> torch.Tensor:
         """The row the next token goes to (``[B, H, 1, D]``); :meth:`commit` takes it in."""
         self._room_for_one(min_cap)
-        return self.buf[:, :, self.end:self.end + 1]
+        return self.buf.narrow(2, self.end, 1)
 
     def commit(self) -> None:
         self.end += 1
@@ -490,6 +490,8 @@ class MuZeroCacheLayer:
         if not self.is_initialized or self.keys is None or self.values is None:
             return
         k_out, v_out = self._flush_lengths(decode_flush)
+        if not k_out and not v_out:
+            return
         keys = self.keys[:, :, :k_out] if k_out else None
         values = self.values[:, :, :v_out] if v_out else None
         if k_out and v_out and self.nbits != 4 and self._alphas["key"] is None and self._alphas["value"] is None:

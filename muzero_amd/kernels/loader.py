@@ -280,16 +280,18 @@ def prepare_mask(attention_mask: torch.Tensor | None, batch: int, length: int) -
         return None
     m = attention_mask
     if m.dim() == 4:
-        m = m[:, 0, -1, :length]
-    elif m.dim() == 2:
-        m = m[:, :length]
-    else:
+        m = m.select(1, 0).select(1, -1)
+    elif m.dim() != 2:
         raise MuZeroHipError(f"unsupported attention mask rank {attention_mask.dim()}")
-    _require(m.shape[-1] == length, f"mask covers {m.shape[-1]} positions, cache holds {length}")
+    _require(m.shape[1] >= length, f"mask covers {m.shape[1]} positions, cache holds {length}")
+    if m.shape[1] != length:
+        m = m.narrow(1, 0, length)
     if m.dtype == torch.bool:
         m = torch.zeros(m.shape, dtype=torch.float32, device=m.device).masked_fill_(~m, float("-inf"))
-    m = m.to(torch.float32).expand(batch, length).contiguous()
-    return m
+    m = m.to(torch.float32)
+    if m.shape[0] != batch:
+        m = m.expand(batch, length)
+    return m.contiguous()
 
 
 # muzero_decode_kernel() -> name
@@ -471,47 +473,70 @@ class DecodePlan:
 
 
 class StepDecode:
-    """A validated :class:`DecodePlan` re-launched for later decode steps of the same
-    cache layer: the caller guarantees (through ``key``) that every tensor the plan
-    points into is the same storage with the same strides, so only the query, the
-    prefix/residual lengths, the output and the workspace size change."""
+    """The validated arguments of a :class:`DecodePlan` or :class:`UnfusedPlan`, re-launched for later decode
+    steps of the same cache layer: the caller guarantees (through ``key``) that every tensor the plan points
+    into is the same storage with the same strides, so only the query, the mask, the prefix / residual
+    lengths, the output and the workspace size change.  A step is one ctypes call; the workspace size and the
+    kernel are asked for again only when the lengths they depend on change."""
 
     __slots__ = ("key", "args", "argp", "lib", "device", "q_dtype", "out_shape", "workspace", "_keep",
-                 "_keep_query", "uses_fold", "kernel")
+                 "_keep_query", "uses_fold", "kernel", "_sized_for", "_run", "_need", "_tile", "_align")
 
-    def __init__(self, plan: DecodePlan, key):
+    def __init__(self, plan, key):
         self.key = key
         self.args = plan.args
         self.argp = ctypes.byref(plan.args)
-        self.lib = plan._lib
+        self.lib = lib = plan._lib
         self.device = plan.device
         self.q_dtype = plan.out.dtype
         self.out_shape = tuple(plan.out.shape)
         self.workspace = plan.workspace
         self._keep = plan._keep  # tables, packed/residual views: kept alive with the arguments
-        self.uses_fold = plan.uses_fold
         self.kernel = plan.kernel
+        self.uses_fold = plan.kernel == "fold"
+        fused = plan.kernel is not None
+        self._run = lib.muzero_decode_attention if fused else lib.muzero_decode_unfused
+        self._need = (lambda argp: lib.muzero_decode_workspace_bytes(argp, None)) if fused else \
+            lib.muzero_decode_unfused_workspace_bytes
+        self._tile = GROUP if fused else 1  # residual tokens that share a workspace size
+        self._align = 16 if fused else 1    # bytes the query rows are aligned to
+        self._sized_for = None
 
-    def launch(self, query: torch.Tensor, n_groups: int, n_residual: int) -> torch.Tensor:
+    def _size(self, n_groups: int, n_residual: int) -> None:
         a = self.args
-        q = query
-        if q.data_ptr() % 16 or q.stride(0) != a.q_sb or q.stride(1) != a.q_sh or q.stride(3) != 1:
-            q = query.contiguous()  # as the plan did (the key pins the query's layout)
-            _require(q.stride(0) == a.q_sb and q.stride(1) == a.q_sh, "query layout changed")
-        a.query = q.data_ptr()
-        a.n_groups, a.n_residual = int(n_groups), int(n_residual)
-        out = torch.empty(self.out_shape, dtype=self.q_dtype, device=self.device)
-        a.out = out.data_ptr()
-        need = self.lib.muzero_decode_workspace_bytes(self.argp, None)
+        need = self._need(self.argp)
         _require(need >= 0, "decode arguments rejected")
         if need > a.workspace_bytes:
             self.workspace = torch.empty((need + 3) // 4, dtype=torch.float32, device=self.device)
             a.workspace = self.workspace.data_ptr()
-        a.workspace_bytes = max(int(need), int(a.workspace_bytes))
-        self.kernel = DECODE_KERNELS[self.lib.muzero_decode_kernel(self.argp)]
-        self.uses_fold = self.kernel == "fold"
-        check(self.lib.muzero_decode_attention(self.argp, stream_ptr(self.device)), "muzero_decode_attention")
-        self._keep_query = q  # alive until the next launch (the kernel reads it asynchronously)
+            a.workspace_bytes = need
+        if self.kernel is not None:
+            self.kernel = DECODE_KERNELS[self.lib.muzero_decode_kernel(self.argp)]
+            self.uses_fold = self.kernel == "fold"
+
+    def launch(self, query: torch.Tensor, n_groups: int, n_residual: int,
+               mask: torch.Tensor | None = None) -> torch.Tensor:
+        a = self.args
+        q = query
+        address = q.data_ptr()
+        if address % self._align or q.stride(0) != a.q_sb or q.stride(1) != a.q_sh or q.stride(3) != 1:
+            q = query.contiguous()  # as the plan did (the key pins the query's layout)
+            _require(q.stride(0) == a.q_sb and q.stride(1) == a.q_sh, "query layout changed")
+            address = q.data_ptr()
+        a.query = address
+        a.n_groups, a.n_residual = n_groups, n_residual
+        if mask is not None:
+            a.mask, a.mask_sb = mask.data_ptr(), mask.stride(0)
+        out = torch.empty(self.out_shape, dtype=self.q_dtype, device=self.device)
+        a.out = out.data_ptr()
+        sized_for = (n_groups, -(-n_residual // self._tile))
+        if sized_for != self._sized_for:
+            self._size(n_groups, n_residual)
+            self._sized_for = sized_for
+        status = self._run(self.argp, stream_ptr(self.device))
+        if status:
+            check(status, "decode")
+        self._keep_query = q, mask  # alive until the next launch (the kernel reads them asynchronously)
         return out
 
 
@@ -533,21 +558,21 @@ def decode_prologue(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torc
              and cos.stride(-1) == sin.stride(-1) == 1 and cos.stride() == sin.stride(), "prologue layouts")
     _require((q_norm_w is None) == (k_norm_w is None), "q_norm and k_norm go together")
     out = torch.empty((b, hq, 1, d), dtype=q.dtype, device=q.device)
-    a = _lib.PrologueArgs()
-    a.batch, a.q_heads, a.kv_heads, a.head_dim, a.io_dtype = b, hq, hkv, d, DTYPE_ENUM[q.dtype]
-    a.q, a.q_sb, a.q_sh = q.data_ptr(), q.stride(0), q.stride(1)
-    a.k, a.k_sb, a.k_sh = k.data_ptr(), k.stride(0), k.stride(1)
-    a.v, a.v_sb, a.v_sh = v.data_ptr(), v.stride(0), v.stride(1)
-    a.cos, a.sin, a.cs_sb = cos.data_ptr(), sin.data_ptr(), (cos.stride(0) if cos.shape[0] > 1 else 0)
+    qw = kw = None
     if q_norm_w is not None:
         _require(q_norm_w.dtype == k_norm_w.dtype == q.dtype and q_norm_w.is_contiguous()
                  and k_norm_w.is_contiguous(), "norm weights")
-        a.q_norm_w, a.k_norm_w = q_norm_w.data_ptr(), k_norm_w.data_ptr()
-    a.eps = float(eps)
-    a.q_out, a.qo_sb, a.qo_sh = out.data_ptr(), out.stride(0), out.stride(1)
-    a.k_dst, a.kd_sb, a.kd_sh = k_dst.data_ptr(), k_dst.stride(0), k_dst.stride(1)
-    a.v_dst, a.vd_sb, a.vd_sh = v_dst.data_ptr(), v_dst.stride(0), v_dst.stride(1)
-    check(load().muzero_decode_prologue(ctypes.byref(a), stream_ptr(q.device)), "muzero_decode_prologue")
+        qw, kw = q_norm_w.data_ptr(), k_norm_w.data_ptr()
+    qs, ks, vs, kd, vd = q.stride(), k.stride(), v.stride(), k_dst.stride(), v_dst.stride()
+    a = _lib.PrologueArgs(
+        b, hq, hkv, d, DTYPE_ENUM[q.dtype],
+        q.data_ptr(), qs[0], qs[1], k.data_ptr(), ks[0], ks[1], v.data_ptr(), vs[0], vs[1],
+        cos.data_ptr(), sin.data_ptr(), cos.stride(0) if cos.shape[0] > 1 else 0,
+        qw, kw, float(eps), out.data_ptr(), hq * d, d,
+        k_dst.data_ptr(), kd[0], kd[1], v_dst.data_ptr(), vd[0], vd[1])
+    status = load().muzero_decode_prologue(ctypes.byref(a), stream_ptr(q.device))
+    if status:
+        check(status, "muzero_decode_prologue")
     return out
 
 
@@ -732,7 +757,7 @@ def mu_zero_av_cuda(attn_weights: torch.Tensor, packed_q: torch.Tensor, mn: torc
 
 
 def unfused_decode_ok(query: torch.Tensor, k_res: torch.Tensor | None, v_res: torch.Tensor | None, n_rep: int) -> bool:
-    """Whether :func:`mu_zero_decode_unfused_hip` takes a decode call of these tensors."""
+    """Whether :class:`UnfusedPlan` takes a decode call of these tensors."""
     return (query.is_cuda and query.dim() == 4 and query.dtype in DTYPE_ENUM and query.stride(3) == 1
             and query.shape[3] <= 256 and 1 <= n_rep <= 16 and 0 < query.shape[0] <= 65535
             and all(t is None or (t.is_cuda and t.device == query.device and t.dtype == query.dtype and t.stride(3) == 1
@@ -741,61 +766,71 @@ def unfused_decode_ok(query: torch.Tensor, k_res: torch.Tensor | None, v_res: to
             and query.shape[1] % n_rep == 0)
 
 
-def mu_zero_decode_unfused_hip(query: torch.Tensor, *, bits: int, n_groups: int, value_prefix: int,
-                               k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res,
-                               alpha_key: float, alpha_value: float, scaling: float,
-                               mask: torch.Tensor | None) -> torch.Tensor:
-    """The reference's default decode of one token (``muzero_decode_unfused``): qk with the residual's logits,
-    softmax, av with the residual's weighted sum.  ``query [B, Hq, 1, D]`` (bf16, fp16, fp32), the packed prefix
-    and the residual as :class:`DecodePlan` takes them, ``mask`` additive fp32 ``[B, L]`` or None; returns
-    ``[B, 1, Hq, D]`` in the query dtype (reference ``attention.py:179-295``)."""
-    dev = _on_gpu(query, k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res, mask)
-    b, hq, _, d = query.shape
-    r = 0 if k_res is None else k_res.shape[2]
-    length, qb, ng = GROUP * n_groups + r, _qbytes(bits), (d + GROUP - 1) // GROUP
-    hkv = (k_res if k_res is not None else k_packed).shape[1]
-    a = _lib.DecodeArgs()
-    if n_groups > 0:
-        mn, sc = _meta4(k_mn, "K min"), _meta4(k_scale, "K scale")
-        _require(k_packed.dtype == torch.uint8 and k_packed.shape[:2] == (b, hkv) and k_packed.shape[2] >= n_groups
-                 and tuple(k_packed.shape[3:]) == (d, qb) and k_packed.stride()[2:] == (d * qb, qb, 1), "packed K layout")
-        _require(mn.shape == sc.shape and mn.shape[:2] == (b, hkv) and mn.shape[2] >= n_groups and mn.shape[3] == d
-                 and mn.dtype == sc.dtype and mn.stride() == sc.stride() and mn.stride()[2:] == (d, 1), "K meta layout")
-        a.meta_dtype = DTYPE_ENUM[mn.dtype]
-        a.k_packed, a.kp_sb, a.kp_sh = ptr(k_packed), k_packed.stride(0), k_packed.stride(1)
-        a.k_mn, a.k_scale, a.km_sb, a.km_sh = ptr(mn), ptr(sc), mn.stride(0), mn.stride(1)
-        a.e_key = ptr(tables.device_table("expm1", alpha_key, dev))
-    if value_prefix > 0:
-        mn, sc = _meta4(v_mn, "V min"), _meta4(v_scale, "V scale")
-        _require(v_packed.dtype == torch.uint8 and v_packed.shape[:2] == (b, hkv) and v_packed.shape[2] >= value_prefix
-                 and tuple(v_packed.shape[3:]) == (ng, qb) and v_packed.stride()[2:] == (ng * qb, qb, 1), "packed V layout")
-        _require(mn.shape == sc.shape and mn.shape[:2] == (b, hkv) and mn.shape[2] >= value_prefix and mn.shape[3] == ng
-                 and mn.dtype == sc.dtype and mn.stride() == sc.stride() and mn.stride()[2:] == (ng, 1), "V meta layout")
-        _require(n_groups == 0 or a.meta_dtype == DTYPE_ENUM[mn.dtype], "meta dtypes")
-        a.meta_dtype = DTYPE_ENUM[mn.dtype]
-        a.v_packed, a.vp_sb, a.vp_sh = ptr(v_packed), v_packed.stride(0), v_packed.stride(1)
-        a.v_mn, a.v_scale, a.vm_sb, a.vm_sh = ptr(mn), ptr(sc), mn.stride(0), mn.stride(1)
-        a.e_value = ptr(tables.device_table("expm1", alpha_value, dev))
-    _require(GROUP * n_groups <= value_prefix <= length, "value_prefix must lie between the key prefix and the cache's end")
-    a.v_prefix = value_prefix if value_prefix != GROUP * n_groups else 0
-    if r > 0:
-        n_v = length - value_prefix
-        _require(v_res is not None and v_res.shape[2] >= n_v, "residual K/V lengths differ")
-        a.k_res, a.kr_sb, a.kr_sh, a.kr_st = ptr(k_res), k_res.stride(0), k_res.stride(1), k_res.stride(2)
-        a.v_res, a.vr_sb, a.vr_sh, a.vr_st = ptr(v_res), v_res.stride(0), v_res.stride(1), v_res.stride(2)
-    if mask is not None:
-        a.mask, a.mask_sb = ptr(mask), mask.stride(0)
-    out = torch.empty((b, 1, hq, d), dtype=query.dtype, device=dev)
-    a.batch, a.kv_heads, a.n_rep, a.head_dim, a.bits = b, hkv, hq // hkv, d, int(bits)
-    a.n_groups, a.n_residual = int(n_groups), int(r)
-    a.io_dtype = a.out_dtype = DTYPE_ENUM[query.dtype]
-    a.scaling = float(scaling)
-    a.query, a.q_sb, a.q_sh = ptr(query), query.stride(0), query.stride(1)
-    a.out, a.out_sb, a.out_sh = ptr(out), out.stride(0), out.stride(2)
-    lib, argp = load(), ctypes.byref(a)
-    need = lib.muzero_decode_unfused_workspace_bytes(argp)
-    _require(need >= 0, "unfused decode arguments rejected")
-    workspace = torch.empty(need, dtype=torch.uint8, device=dev)
-    a.workspace, a.workspace_bytes = ptr(workspace), need
-    check(lib.muzero_decode_unfused(argp, stream_ptr(dev)), "muzero_decode_unfused")
-    return out
+class UnfusedPlan:
+    """The reference's default decode of one token (``muzero_decode_unfused``), validated and ready to launch:
+    qk with the residual's logits, softmax, av with the residual's weighted sum.  ``query [B, Hq, 1, D]`` (bf16,
+    fp16, fp32), the packed prefix and the residual as :class:`DecodePlan` takes them, ``mask`` additive fp32
+    ``[B, L]`` or None; :meth:`run` returns ``[B, 1, Hq, D]`` in the query dtype (reference
+    ``attention.py:179-295``)."""
+
+    kernel = None  # none of the fused kernels
+
+    def __init__(self, query: torch.Tensor, *, bits: int, n_groups: int, value_prefix: int,
+                 k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res,
+                 alpha_key: float, alpha_value: float, scaling: float, mask: torch.Tensor | None):
+        dev = _on_gpu(query, k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res, mask)
+        b, hq, _, d = query.shape
+        r = 0 if k_res is None else k_res.shape[2]
+        length, qb, ng = GROUP * n_groups + r, _qbytes(bits), (d + GROUP - 1) // GROUP
+        hkv = (k_res if k_res is not None else k_packed).shape[1]
+        a = _lib.DecodeArgs()
+        if n_groups > 0:
+            mn, sc = _meta4(k_mn, "K min"), _meta4(k_scale, "K scale")
+            _require(k_packed.dtype == torch.uint8 and k_packed.shape[:2] == (b, hkv) and k_packed.shape[2] >= n_groups
+                     and tuple(k_packed.shape[3:]) == (d, qb) and k_packed.stride()[2:] == (d * qb, qb, 1), "packed K layout")
+            _require(mn.shape == sc.shape and mn.shape[:2] == (b, hkv) and mn.shape[2] >= n_groups and mn.shape[3] == d
+                     and mn.dtype == sc.dtype and mn.stride() == sc.stride() and mn.stride()[2:] == (d, 1), "K meta layout")
+            a.meta_dtype = DTYPE_ENUM[mn.dtype]
+            a.k_packed, a.kp_sb, a.kp_sh = ptr(k_packed), k_packed.stride(0), k_packed.stride(1)
+            a.k_mn, a.k_scale, a.km_sb, a.km_sh = ptr(mn), ptr(sc), mn.stride(0), mn.stride(1)
+            a.e_key = ptr(tables.device_table("expm1", alpha_key, dev))
+        if value_prefix > 0:
+            mn, sc = _meta4(v_mn, "V min"), _meta4(v_scale, "V scale")
+            _require(v_packed.dtype == torch.uint8 and v_packed.shape[:2] == (b, hkv) and v_packed.shape[2] >= value_prefix
+                     and tuple(v_packed.shape[3:]) == (ng, qb) and v_packed.stride()[2:] == (ng * qb, qb, 1), "packed V layout")
+            _require(mn.shape == sc.shape and mn.shape[:2] == (b, hkv) and mn.shape[2] >= value_prefix and mn.shape[3] == ng
+                     and mn.dtype == sc.dtype and mn.stride() == sc.stride() and mn.stride()[2:] == (ng, 1), "V meta layout")
+            _require(n_groups == 0 or a.meta_dtype == DTYPE_ENUM[mn.dtype], "meta dtypes")
+            a.meta_dtype = DTYPE_ENUM[mn.dtype]
+            a.v_packed, a.vp_sb, a.vp_sh = ptr(v_packed), v_packed.stride(0), v_packed.stride(1)
+            a.v_mn, a.v_scale, a.vm_sb, a.vm_sh = ptr(mn), ptr(sc), mn.stride(0), mn.stride(1)
+            a.e_value = ptr(tables.device_table("expm1", alpha_value, dev))
+        _require(GROUP * n_groups <= value_prefix <= length, "value_prefix must lie between the key prefix and the cache's end")
+        a.v_prefix = value_prefix if value_prefix != GROUP * n_groups else 0
+        if r > 0:
+            n_v = length - value_prefix
+            _require(v_res is not None and v_res.shape[2] >= n_v, "residual K/V lengths differ")
+            a.k_res, a.kr_sb, a.kr_sh, a.kr_st = ptr(k_res), k_res.stride(0), k_res.stride(1), k_res.stride(2)
+            a.v_res, a.vr_sb, a.vr_sh, a.vr_st = ptr(v_res), v_res.stride(0), v_res.stride(1), v_res.stride(2)
+        if mask is not None:
+            a.mask, a.mask_sb = ptr(mask), mask.stride(0)
+        out = torch.empty((b, 1, hq, d), dtype=query.dtype, device=dev)
+        a.batch, a.kv_heads, a.n_rep, a.head_dim, a.bits = b, hkv, hq // hkv, d, int(bits)
+        a.n_groups, a.n_residual = int(n_groups), int(r)
+        a.io_dtype = a.out_dtype = DTYPE_ENUM[query.dtype]
+        a.scaling = float(scaling)
+        a.query, a.q_sb, a.q_sh = ptr(query), query.stride(0), query.stride(1)
+        a.out, a.out_sb, a.out_sh = ptr(out), out.stride(0), out.stride(2)
+        lib = load()
+        need = lib.muzero_decode_unfused_workspace_bytes(ctypes.byref(a))
+        _require(need >= 0, "unfused decode arguments rejected")
+        ws = torch.empty((need + 3) // 4, dtype=torch.float32, device=dev)
+        a.workspace, a.workspace_bytes = ptr(ws), need
+        self.args, self.device, self.out, self.workspace, self._lib = a, dev, out, ws, lib
+        # tables are held by the library's cache; everything else the arguments point into by these references
+        self._keep = [query, k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res, mask]
+
+    def run(self) -> torch.Tensor:
+        check(self._lib.muzero_decode_unfused(ctypes.byref(self.args), stream_ptr(self.device)),
+              "muzero_decode_unfused")
+        return self.out

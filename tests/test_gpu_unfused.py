@@ -32,10 +32,11 @@ def _both(B, hkv, n_rep, d, tokens, bits, dtype, residual=128, mask=False, logq=
     if mask:
         m = torch.zeros(B, 1, 1, tokens, dtype=dtype, device="cuda")
         m[0, ..., :tokens // 3] = torch.finfo(dtype).min
-    pre = st["key_prefix_length"], st["value_prefix_length"], layer.keys, layer.values, 2.0, 2.0
-    got = A._split_launches(layer, _Module(n_rep), q, m, d ** -0.5, *pre)
-    prepared = A._k.prepare_mask(m, B, tokens)
-    want = A._split_steps(layer, n_rep, q, prepared, d ** -0.5, *pre)
+    got = mz.mu_zero_decode_attention_forward(_Module(n_rep), q, m, d ** -0.5, st)[0]
+    again = mz.mu_zero_decode_attention_forward(_Module(n_rep), q.clone(), m, d ** -0.5, st)[0]  # the cached arguments
+    assert torch.equal(got.view(torch.uint8), again.view(torch.uint8))
+    want = A._split_steps(layer, n_rep, q, A._k.prepare_mask(m, B, tokens), d ** -0.5, st["key_prefix_length"],
+                          st["value_prefix_length"], layer.keys, layer.values, 2.0, 2.0)
     return got, want
 
 
