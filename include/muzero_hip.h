@@ -136,6 +136,18 @@ int muzero_dequantize_keys(const mz_dequant_args* args, mz_stream_t stream);
 int muzero_dequantize_values(const mz_dequant_args* args, mz_stream_t stream);
 
 /*
+ * Quantize and dequantize a tensor x [B, H, T, D] (last dim contiguous) without storing the codes: the
+ * offline round trip (muzero/quantizer.py:273-323).  keys != 0: groups of 64 tokens per channel (T a multiple
+ * of 64); else groups of 64 channels per token, the last one zero-filled.  Groups are quantized from fp32,
+ * min / scale rounded to meta_dtype, the result written to out (same shape and dtype as x).  table: the
+ * fp32 threshold table of the alpha (as muzero_quantize_rows takes it for fp32 rows), e_table its expm1 rows.
+ */
+int muzero_roundtrip(const void* x, int dtype, int keys, int B, int H, int T, int D, int64_t x_sb, int64_t x_sh,
+                     int64_t x_st, void* out, int64_t o_sb, int64_t o_sh, int64_t o_st,
+                     int meta_dtype, int bits, float eps, const void* table, const float* e_table,
+                     mz_stream_t stream);
+
+/*
  * Alpha statistics of a block x [B, H, T, D] (last dim contiguous), as the cache
  * flattens it into rows (muzero/quantizer.py:46-55, muzero/cache/layer.py:223-301).
  * keys != 0: groups of 64 tokens per channel, in order (b, h, t/64, d) (T a multiple

@@ -146,6 +146,8 @@ SIGNATURES = {
                                        c_int, c_vp, c_vp]),
     "muzero_dequantize_keys": (c_int, [ctypes.POINTER(DequantArgs), c_vp]),
     "muzero_dequantize_values": (c_int, [ctypes.POINTER(DequantArgs), c_vp]),
+    "muzero_roundtrip": (c_int, [c_vp, c_int, c_int, c_int, c_int, c_int, c_int, c_i64, c_i64, c_i64,
+                                 c_vp, c_i64, c_i64, c_i64, c_int, c_int, c_float, c_vp, c_vp, c_vp]),
     "muzero_block_stats": (c_int, [c_vp, c_int, c_int, c_int, c_int, c_int, c_int, c_i64, c_i64, c_i64,
                                    c_vp, c_vp, c_i64, c_i64, c_vp]),
     "muzero_select3": (c_int, [c_vp, c_int, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp]),

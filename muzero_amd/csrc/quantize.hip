@@ -12,303 +12,19 @@
 // packs and stores its own bytes and a wave's stores are contiguous.  The grid
 // is persistent (a few workgroups per CU loop over the groups), so each
 // workgroup stages the table once.
-#include "common.hpp"
+#include "quantize_core.hpp"
 
 #include <algorithm>
 #include <type_traits>
 
 namespace mz {
 
-constexpr int QWG = 256;  // threads per quantize workgroup
 // Values per lane: each lane quantizes 32 values of a 64-value group (two
 // lanes per group), so a wave quantizes 32 groups and a group's parameters
 // are formed once per 32 values.  Key groups read their column from an LDS
 // tile.
 constexpr int QN_ROWS = 32;
 constexpr int QN_KEYS = 32;
-
-// Compander parameters of one group (quantizer.py:169-181), every op rounded
-// to the input dtype DT.
-struct QParams {
-  float mn, sc, za, zl, pb, nb, pe, ne, eps;
-  float rsc, rpe, rne;  // v_rcp_f32 of sc, pe, ne (16-bit inputs only)
-  float ea, ec;         // fp32 inputs: the table's alpha estimate and 1 / log2(1 + ea) (see code_offset_f32)
-};
-
-// rnd<DT>(a / b) for a, b values of the 16-bit input dtype, given r = rcp(b).
-// bf16: a and b have 8-bit significands, so a / b is never a bf16 rounding
-// midpoint and lies at least 2^7 fp32 ulps from one (a = b * odd 9-bit
-// significand is impossible; the distance is >= 1/B bf16 half-ulps with the
-// odd part B < 2^8); a * rcp(b) is within 3 ulps, so rounding it to bf16 gives
-// the reference's round(fp32 division).  fp16 (11-bit significands, distance
-// >= 2 ulps) takes one residual correction (< 1 ulp) except where b is 0 or
-// inf, where a * rcp(b) is already the IEEE quotient (inf, NaN or 0).  rcp of
-// a b above 2^126 would be denormal: such groups use the IEEE division.
-template <int DT, bool FAST>
-__device__ __forceinline__ float qdiv(float a, float b, float r) {
-  if constexpr (DT == MZ_F32 || !FAST) {
-    return rnd<DT>(a / b);
-  } else if constexpr (DT == MZ_BF16) {
-    return rnd<DT>(a * r);
-  } else {
-    const float q0 = a * r;
-    const float q1 = fmaf(fmaf(-b, q0, a), r, q0);
-    return rnd<DT>((b != 0.f && b != __builtin_inff()) ? q1 : q0);
-  }
-}
-
-// Whether the reciprocal form applies to every division of the group.
-template <int DT>
-__device__ __forceinline__ bool qfast(const struct QParams& g) {
-  if constexpr (DT == MZ_F16) return true;  // an fp16 scale is <= 65504 or inf
-  return DT != MZ_F32 && !(g.sc > 0x1p126f && g.sc < __builtin_inff());
-}
-
-template <int DT, int BITS>
-__device__ __forceinline__ QParams qparams(float mn, float mx, float eps_in) {
-  constexpr float qmax = (float)((1 << BITS) - 1);
-  QParams g;
-  g.eps = rnd<DT>(eps_in);
-  g.mn = mn;
-  g.sc = clamp_min(rnd<DT>(mx - mn), g.eps);
-  if constexpr (DT == MZ_BF16) {
-    // the reciprocal form of the division (exact for bf16 operands, see
-    // qdiv) unless the scale's reciprocal would be denormal; the IEEE
-    // division runs only in a wave that holds such a group
-    g.rsc = __builtin_amdgcn_rcpf(g.sc);
-    const float a = rnd<DT>(0.f - mn);
-    float zq = rnd<DT>(a * g.rsc);
-    const bool slow = g.sc > 0x1p126f && g.sc < __builtin_inff();
-    if (__ballot(slow) != 0) {
-      if (slow) zq = rnd<DT>(a / g.sc);
-    }
-    g.za = clamp01(zq);
-  } else {
-    g.za = clamp01(rnd<DT>(rnd<DT>(0.f - mn) / g.sc));
-  }
-  g.zl = rintf(rnd<DT>(g.za * qmax));
-  g.pb = clamp_min(rnd<DT>(qmax - g.zl), 1.f);
-  g.nb = clamp_min(g.zl, 1.f);
-  g.pe = clamp_min(rnd<DT>(1.f - g.za), g.eps);
-  g.ne = clamp_min(g.za, g.eps);
-  if constexpr (DT != MZ_F32) {
-    if constexpr (DT != MZ_BF16) g.rsc = __builtin_amdgcn_rcpf(g.sc);
-    g.rpe = __builtin_amdgcn_rcpf(g.pe);
-    g.rne = __builtin_amdgcn_rcpf(g.ne);
-  }
-  return g;
-}
-
-// Compander table in LDS: fp32 inputs use the threshold rows of bins 1..qmax
-// (#{k : p >= T[bins][k]}, binary search); bf16/fp16 inputs the 16-bit ratio
-// table indexed by the pattern of p.  Table bytes staged per workgroup:
-template <int DT, int BITS>
-struct QTable {
-  static constexpr int QMAX = (1 << BITS) - 1;
-  static constexpr int BYTES = DT == MZ_F32 ? QMAX * (QMAX + 1) / 2 * 4
-                                            : ((DT == MZ_BF16 ? 0x3F80 : 0x3C00) + 1) * 2;
-  static constexpr bool IN_LDS = BYTES <= 40 * 1024;  // 8-bit fp32 thresholds (128 KB) stay in global memory
-  static constexpr int LDS_BYTES = IN_LDS ? (BYTES + 15) / 16 * 16 : 16;
-};
-
-template <int DT, int BITS>
-__device__ __forceinline__ void stage_table(uint8_t* lds, const void* table) {
-  using TB = QTable<DT, BITS>;
-  if constexpr (TB::IN_LDS) {
-    const uint16_t* src = (const uint16_t*)table;
-    for (int i = threadIdx.x; i < TB::BYTES / 2; i += QWG) ((uint16_t*)lds)[i] = src[i];
-    __syncthreads();
-  }
-}
-
-// fp32 inputs: the code offset #{k in 1..bins : row[k-1] <= p} of a
-// normalised distance p over the threshold row of `bins` (monotone: the
-// offset is the reference's round(log1p(alpha*p) / lb * bins), tables.py).
-// An estimate from the hardware log2 (bins * log2(1 + ea*p) * ec, ea the
-// alpha the row of bins 1 implies) is within one of it; four independent
-// reads of the thresholds around it give the count, and two of them check
-// that the estimate's window [k0, k0 + 2] holds it (every threshold up to
-// k0 at or below p, the one after k0 + 2 above).  Where the check fails the
-// binary search runs, so the result is exact whatever the estimate.  Used
-// from 5 bits (rows of up to 31 .. 255 thresholds: 5 to 8 dependent reads
-// of the binary search); 8-bit keys / values 1.65x / 2.3x faster.
-__device__ __forceinline__ int code_offset_f32(const float* row, int bins, float p, const QParams& g) {
-  const float e = (float)bins * __builtin_amdgcn_logf(fmaf(g.ea, p, 1.f)) * g.ec;
-  const float r = rintf(e) - 1.f;
-  const int k0 = (int)__builtin_amdgcn_fmed3f(r == r ? r : 0.f, 0.f, (float)max(bins - 2, 0));
-  // row[k0 - 1 .. k0 + 2], each index kept inside the row (an entry outside
-  // it is not used: its test is decided by the bounds instead)
-  const float t0 = row[max(k0 - 1, 0)], t1 = row[min(k0, bins - 1)], t2 = row[min(k0 + 1, bins - 1)],
-              t3 = row[min(k0 + 2, bins - 1)];
-  const bool below = k0 == 0 || t0 <= p;         // thresholds 1..k0 at or below p
-  const bool above = k0 + 3 > bins || t3 > p;    // thresholds k0 + 3.. above p
-  const int cnt = k0 + (k0 + 1 <= bins && t1 <= p ? 1 : 0) + (k0 + 2 <= bins && t2 <= p ? 1 : 0);
-  if (below && above) return cnt;
-  int lo = 0, hi = bins;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (row[mid] <= p) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
-
-// Code of one value given its group's parameters (quantizer.py:172-184).
-// FINITE: the group's mn and scale are finite and every divisor (scale, pe,
-// ne) is positive, so no intermediate is NaN or infinite and every clamped
-// quantity is >= 0 (v >= mn; the side's offset from za is >= 0): the NaN
-// cases and the lower clamps drop out and give the same results.
-template <int DT, int BITS, bool FAST, bool FINITE>
-__device__ __forceinline__ uint32_t value_code(float v, const QParams& g, const uint8_t* lds, const void* table) {
-  constexpr float qmax = (float)((1 << BITS) - 1);
-  const float n0 = qdiv<DT, FAST>(rnd<DT>(v - g.mn), g.sc, g.rsc);
-  const float norm = FINITE ? fminf(n0, 1.f) : clamp01(n0);
-  const bool up = norm >= g.za;  // torch.where(norm >= za, q_pos, q_neg); false on NaN
-  // Only the selected side is evaluated: operands are chosen before the one
-  // division, which computes exactly what the unselected-branch form would.
-  const float p0 = qdiv<DT, FAST>(rnd<DT>(up ? norm - g.za : g.za - norm), up ? g.pe : g.ne, up ? g.rpe : g.rne);
-  const float p = FINITE ? fminf(p0, 1.f) : clamp01(p0);
-  const float bins = up ? g.pb : g.nb;
-  float off;
-  if constexpr (DT == MZ_F32) {
-    const float* T = QTable<DT, BITS>::IN_LDS ? (const float*)lds : (const float*)table;
-    const int ib = (FINITE || bins == bins) ? (int)bins : 1;
-    const float* row = T + ib * (ib - 1) / 2;
-    int lo;
-    if constexpr (BITS >= 5) {
-      lo = code_offset_f32(row, ib, p, g);
-    } else {
-      // up to 15 thresholds a row: the binary search's 4 steps measured as fast as the estimate
-      lo = 0;
-      int hi = ib;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (row[mid] <= p) lo = mid + 1; else hi = mid;
-      }
-    }
-    off = (FINITE || p == p) ? (float)lo : __builtin_nanf("");
-  } else {
-    const uint16_t* Y = (const uint16_t*)lds;
-    float y;
-    if (FINITE || p == p) {
-      const uint32_t pat = (DT == MZ_BF16 ? (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)p)  // p is not NaN
-                                          : (uint32_t)f2h(p)) & 0x7FFFu;                          // -0 -> 0
-      y = DT == MZ_BF16 ? bf2f(Y[pat]) : h2f(Y[pat]);
-    } else {
-      y = p;
-    }
-    off = rintf(rnd<DT>(y * bins));
-  }
-  // zl +- off is an integer in [-1, qmax + 1] <= 256 there: exact in every
-  // input dtype, so its rounding is the identity
-  const float q = FINITE ? (up ? g.zl + off : g.zl - off) : rnd<DT>(up ? g.zl + off : g.zl - off);
-  // clamp(0, qmax).to(uint8); a NaN code converts to 0 (as on the reference CPU)
-  if (!FINITE && !(q == q)) return 0u;
-  return (uint32_t)fminf(fmaxf(q, 0.f), qmax);
-}
-
-// value_code<MZ_BF16, BITS, true, true> of two values at once (the two
-// chains interleave; each rounding to bf16 is one v_cvt_pk_bf16_f32).
-typedef float f32x2v __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void rnd_bf16_pair(float& a, float& b) {
-  a = rnd<MZ_BF16>(a);
-  b = rnd<MZ_BF16>(b);
-}
-
-//
-// The same values as the op-by-op chain, in fewer ops (every rewrite below is
-// exact for a finite group: mn and the scale finite, the divisors positive):
-//  - min(rnd(x), 1) = rnd(min(x, 1)) (1 is a bf16 value and rounding is
-//    monotone), and x >= 0, so the clamp rides on the multiply (med3 = the
-//    VOP3 clamp bit);
-//  - the selected side's difference, za - n below za and n - za above, is
-//    |n - za| (fp32 negation is exact, and bf16 rounding is symmetric);
-//  - the down side's offset is subtracted: zl - rint(rnd(y * nb)) =
-//    zl + rint(rnd(y * -nb)) (both roundings are symmetric);
-//  - p is a bf16 value >= +0 with a zero low half, so its ratio-table byte
-//    address, pattern * 2, is its bit pattern >> 15.
-template <int BITS>
-__device__ __forceinline__ void value_code_bf16_pair(float v0, float v1, const QParams& g, const uint8_t* lds,
-                                                     uint32_t& c0, uint32_t& c1) {
-  constexpr float qmax = (float)((1 << BITS) - 1);
-  float a0 = v0 - g.mn, a1 = v1 - g.mn;
-  rnd_bf16_pair(a0, a1);
-  float n0 = __builtin_amdgcn_fmed3f(a0 * g.rsc, 0.f, 1.f), n1 = __builtin_amdgcn_fmed3f(a1 * g.rsc, 0.f, 1.f);
-  rnd_bf16_pair(n0, n1);
-  const bool up0 = n0 >= g.za, up1 = n1 >= g.za;
-  float d0 = n0 - g.za, d1 = n1 - g.za;
-  rnd_bf16_pair(d0, d1);  // |rnd(x)| = rnd(|x|): the absolute value rides on the multiply's operand
-  float p0 = __builtin_amdgcn_fmed3f(__builtin_fabsf(d0) * (up0 ? g.rpe : g.rne), 0.f, 1.f);
-  float p1 = __builtin_amdgcn_fmed3f(__builtin_fabsf(d1) * (up1 ? g.rpe : g.rne), 0.f, 1.f);
-  rnd_bf16_pair(p0, p1);
-  const float y0 = bf2f(*(const uint16_t*)(lds + (__float_as_uint(p0) >> 15)));
-  const float y1 = bf2f(*(const uint16_t*)(lds + (__float_as_uint(p1) >> 15)));
-  float o0 = y0 * (up0 ? g.pb : -g.nb), o1 = y1 * (up1 ? g.pb : -g.nb);
-  rnd_bf16_pair(o0, o1);
-  // zl + off: an integer in [-1, qmax + 1], exact in bf16 (its rounding is the identity)
-  const float q0 = g.zl + rintf(o0), q1 = g.zl + rintf(o1);
-  c0 = (uint32_t)__builtin_amdgcn_fmed3f(q0, 0.f, qmax);
-  c1 = (uint32_t)__builtin_amdgcn_fmed3f(q1, 0.f, qmax);
-}
-
-// value_code<MZ_F16, BITS, true, true> with the rewrites of the bf16 pair
-// form, which hold for fp16 as well (they use only that 1 is an fp16 value,
-// that rounding is monotone and symmetric, and that in a finite group every
-// quotient is >= +0).  Each division is a * rcp(b) plus one residual
-// correction (qdiv; b is positive and finite here), the clamp riding on the
-// correction's FMA; p's fp16 pattern addresses the ratio table directly.
-template <int BITS>
-__device__ __forceinline__ uint32_t value_code_f16(float v, const QParams& g, const uint8_t* lds) {
-  constexpr float qmax = (float)((1 << BITS) - 1);
-  const float a = rnd<MZ_F16>(v - g.mn);
-  const float n0 = a * g.rsc;
-  const float n = rnd<MZ_F16>(__builtin_amdgcn_fmed3f(__builtin_fmaf(__builtin_fmaf(-g.sc, n0, a), g.rsc, n0), 0.f, 1.f));
-  const bool up = n >= g.za;
-  const float d = __builtin_fabsf(rnd<MZ_F16>(n - g.za));
-  const float b = up ? g.pe : g.ne, r = up ? g.rpe : g.rne;
-  const float p0 = d * r;
-  const uint32_t pat = f2h(__builtin_amdgcn_fmed3f(__builtin_fmaf(__builtin_fmaf(-b, p0, d), r, p0), 0.f, 1.f));
-  const float y = h2f(*(const uint16_t*)(lds + 2 * (pat & 0x7FFFu)));
-  const float o = rnd<MZ_F16>(y * (up ? g.pb : -g.nb));
-  // zl + off: an integer in [-1, qmax + 1], exact in fp16
-  return (uint32_t)__builtin_amdgcn_fmed3f(g.zl + rintf(o), 0.f, qmax);
-}
-
-// Min / max over the 8 lanes of a group (lanes 8k..8k+7), NaN-propagating:
-// IEEE 754-2019 minimum / maximum (v_minimum3_f32 / v_maximum3_f32), which
-// return NaN when either operand is NaN, as torch's amin / amax do.  (Between
-// -0 and +0 they pick -0 / +0; torch's choice there depends on its
-// vectorisation.  The codes are the same either way: only the sign of a zero
-// minimum or maximum in the metadata can differ.)
-__device__ __forceinline__ float fmin_nan(float a, float b) { return __builtin_elementwise_minimum(a, b); }
-__device__ __forceinline__ float fmax_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
-// Over the L lanes of a group (aligned runs of L = 2, 4 or 8 lanes).
-template <int L>
-__device__ __forceinline__ float group_min(float v) {
-  if constexpr (L >= 2) v = fmin_nan(v, dpp_sel<DPP_QUAD_XOR1>(v));
-  if constexpr (L >= 4) v = fmin_nan(v, dpp_sel<DPP_QUAD_XOR2>(v));
-  if constexpr (L >= 8) v = fmin_nan(v, dpp_sel<DPP_ROW_HALF_MIRROR>(v));
-  return v;
-}
-template <int L>
-__device__ __forceinline__ float group_max(float v) {
-  if constexpr (L >= 2) v = fmax_nan(v, dpp_sel<DPP_QUAD_XOR1>(v));
-  if constexpr (L >= 4) v = fmax_nan(v, dpp_sel<DPP_QUAD_XOR2>(v));
-  if constexpr (L >= 8) v = fmax_nan(v, dpp_sel<DPP_ROW_HALF_MIRROR>(v));
-  return v;
-}
-
-// NaN-propagating min / max of x[0..N) (a balanced tree).
-template <int N, int S = 0>
-__device__ __forceinline__ float tree_min(const float* x) {
-  if constexpr (N == 1) return x[S];
-  else return fmin_nan(tree_min<N / 2, S>(x), tree_min<N / 2, S + N / 2>(x));
-}
-template <int N, int S = 0>
-__device__ __forceinline__ float tree_max(const float* x) {
-  if constexpr (N == 1) return x[S];
-  else return fmax_nan(tree_max<N / 2, S>(x), tree_max<N / 2, S + N / 2>(x));
-}
 
 // Quantize the 8 values x[0..7] of a chunk with the group's parameters and
 // store their BITS packed bytes at dst.
@@ -351,16 +67,6 @@ __device__ __forceinline__ void quantize_chunk8(const float* x, const QParams& g
   }
 }
 
-// The offset estimate's constants (code_offset_f32) from the threshold t of
-// bins 1 (index 0 of the table), where log1p(alpha*t) / lb crosses 1/2:
-// (1 + alpha*t)^2 = 1 + alpha, so alpha = (1 - 2t) / t^2.
-template <int BITS>
-__device__ __forceinline__ void set_estimate(QParams& g, const uint8_t* lds, const void* table) {
-  const float t = (QTable<MZ_F32, BITS>::IN_LDS ? (const float*)lds : (const float*)table)[0];
-  g.ea = (1.f - 2.f * t) / (t * t);
-  g.ec = 1.f / __builtin_amdgcn_logf(1.f + g.ea);
-}
-
 // Quantize this lane's N values x[0..N) (positions N*part .. N*part+N-1 of
 // its group, which 64 / N lanes share) and store its N*BITS/8 packed bytes
 // at prow + part*N*BITS/8; lane part 0 stores the group's metadata at index
@@ -386,27 +92,6 @@ __device__ __forceinline__ void quantize_lane(const float (&x)[N], int part, uin
   if (part == 0) {
     store_val(mn_out, midx, mn, meta_dtype);
     store_val(sc_out, midx, g.sc, meta_dtype);
-  }
-}
-
-// 8 consecutive values at p[i..i+7] (VEC: one or two 16-byte loads).
-template <int DT, bool VEC>
-__device__ __forceinline__ void load8(float (&x)[8], const void* p, int64_t i) {
-  if constexpr (VEC && DT == MZ_F32) {
-    const float4 a = *(const float4*)((const float*)p + i);
-    const float4 b = *(const float4*)((const float*)p + i + 4);
-    x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w, x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
-  } else if constexpr (VEC) {
-    const uint4 a = *(const uint4*)((const uint16_t*)p + i);
-    const uint32_t u[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      x[2 * k] = DT == MZ_BF16 ? bf2f((uint16_t)u[k]) : h2f((uint16_t)u[k]);
-      x[2 * k + 1] = DT == MZ_BF16 ? bf2f((uint16_t)(u[k] >> 16)) : h2f((uint16_t)(u[k] >> 16));
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) x[k] = load_val<DT>(p, i + k);
   }
 }
 

@@ -272,6 +272,31 @@ def dequantize_block(packed: torch.Tensor, mn: torch.Tensor, scale: torch.Tensor
     return out
 
 
+def roundtrip_ok(x: torch.Tensor, kind: str, bits: int, meta_dtype: torch.dtype) -> bool:
+    """Whether :func:`roundtrip_block` takes ``x``."""
+    return (x.is_cuda and type(x) is torch.Tensor and x.dim() == 4 and x.dtype in DTYPE_ENUM
+            and meta_dtype in DTYPE_ENUM and 1 <= bits <= 8 and (kind == "value" or x.shape[2] % GROUP == 0))
+
+
+def roundtrip_block(x: torch.Tensor, kind: str, bits: int, alpha: float, eps: float,
+                    meta_dtype: torch.dtype) -> torch.Tensor:
+    """``x [B, H, T, D]`` quantized from fp32 and dequantized again in one launch (``muzero_roundtrip``):
+    keys grouped per channel over 64 tokens, values per token over 64 channels."""
+    x = x if x.stride(3) == 1 else x.contiguous()
+    b, h, t, d = x.shape
+    dev = x.device
+    out = torch.empty((b, h, t, d), dtype=x.dtype, device=dev)
+    if out.numel() == 0:
+        return out
+    st = load().muzero_roundtrip(ptr(x), DTYPE_ENUM[x.dtype], int(kind == "key"), b, h, t, d,
+                                 x.stride(0), x.stride(1), x.stride(2), ptr(out), h * t * d, t * d, d,
+                                 DTYPE_ENUM[meta_dtype], int(bits), float(eps),
+                                 ptr(tables.quantize_table(alpha, torch.float32, dev)),
+                                 ptr(tables.device_table("expm1", alpha, dev)), stream_ptr(dev))
+    check(st, "muzero_roundtrip")
+    return out
+
+
 # --------------------------------------------------------------------------- decode attention
 
 def prepare_mask(attention_mask: torch.Tensor | None, batch: int, length: int) -> torch.Tensor | None:

@@ -332,7 +332,12 @@ def roundtrip(
         alpha_value = select_alpha(value, bits=bits, q_group_size=q_group_size, kind="value")
 
     g = q_group_size
+    if g == GROUP and amax_eps == 1e-8 and _k.roundtrip_ok(key, "key", bits, amax_dtype) and \
+            _k.roundtrip_ok(value, "value", bits, amax_dtype):
+        return (_k.roundtrip_block(key, "key", bits, float(alpha_key), amax_eps, amax_dtype),
+                _k.roundtrip_block(value, "value", bits, float(alpha_value), amax_eps, amax_dtype))
 
+    # other tensors: row by row (and its errors)
     def codec(rows: torch.Tensor, alpha: float, dtype: torch.dtype) -> torch.Tensor:
         packed, mn, scale = quantize_rows(rows.float(), bits, alpha, amax_eps, amax_dtype)
         return dequantize_rows(packed, mn, scale, bits, alpha, g, dtype, amax_eps=amax_eps)
