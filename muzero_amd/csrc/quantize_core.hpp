@@ -188,18 +188,16 @@ __device__ __forceinline__ uint32_t value_code(float v, const QParams& g, const 
   return (uint32_t)fminf(fmaxf(q, 0.f), qmax);
 }
 
-// value_code<MZ_BF16, BITS, true, true> of two values at once (the two
-// chains interleave; each rounding to bf16 is one v_cvt_pk_bf16_f32).
-typedef float f32x2v __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void rnd_bf16_pair(float& a, float& b) {
-  a = rnd<MZ_BF16>(a);
-  b = rnd<MZ_BF16>(b);
-}
-
+// value_code<MZ_BF16, BITS, true, true> of 8 values (4 dwords) and their packed
+// codes.
 //
 // The same values as the op-by-op chain, in fewer ops (every rewrite below is
 // exact for a finite group: mn and the scale finite, the divisors positive):
+//  - v - mn is one v_dot2_f32_bf16 on the dword as it was loaded: v * 1 + the
+//    other half * 0 - mn.  Its fp32 result may differ from the subtraction's in
+//    the last bit, never in the bf16 it rounds to (checked over all pairs of
+//    finite bf16 values, both halves);
+//  - each rounding to bf16 is one v_cvt_pk_bf16_f32 (rnd);
 //  - min(rnd(x), 1) = rnd(min(x, 1)) (1 is a bf16 value and rounding is
 //    monotone), and x >= 0, so the clamp rides on the multiply (med3 = the
 //    VOP3 clamp bit);
@@ -208,29 +206,74 @@ __device__ __forceinline__ void rnd_bf16_pair(float& a, float& b) {
 //  - the down side's offset is subtracted: zl - rint(rnd(y * nb)) =
 //    zl + rint(rnd(y * -nb)) (both roundings are symmetric);
 //  - p is a bf16 value >= +0 with a zero low half, so its ratio-table byte
-//    address, pattern * 2, is its bit pattern >> 15.
+//    address, pattern * 2, is its bit pattern >> 15;
+//  - y * bins is a v_dot2_f32_bf16 on the table's 16-bit entry (8 bits by 8
+//    bits: exact);
+//  - rint is the addition of M = 1.5 * 2^23, whose sum's low bits are the
+//    integer; the clamp to [0, qmax] is taken on the sum, from M - zl to
+//    M - zl + qmax (exact), and M's and zl's bits leave once per packed word.
+struct BfGroup {
+  float nmn, rsc, za, rpe, rne, lo, hi;
+  uint32_t pb, nb;  // bf16 bits of pb and -nb
+  uint32_t base;    // bits of M - zl, the sum's where the code is 0
+  __device__ __forceinline__ BfGroup(const QParams& g, float qmax)
+      : nmn(-g.mn), rsc(g.rsc), za(g.za), rpe(g.rpe), rne(g.rne), lo(12582912.f - g.zl), hi(12582912.f - g.zl + qmax),
+        pb(__float_as_uint(g.pb) >> 16), nb(__float_as_uint(-g.nb) >> 16), base(__float_as_uint(lo)) {}
+};
+
+// Dot products whose results other instructions read: they wait inside the
+// block (three wait states after a dot, once for eight).
+__device__ __forceinline__ void bf16_sub8(const uint32_t* w, float nmn, float (&a)[8]) {
+  asm("v_dot2_f32_bf16 %0, %8, %12, %14\n\tv_dot2_f32_bf16 %1, %8, %13, %14\n\t"
+      "v_dot2_f32_bf16 %2, %9, %12, %14\n\tv_dot2_f32_bf16 %3, %9, %13, %14\n\t"
+      "v_dot2_f32_bf16 %4, %10, %12, %14\n\tv_dot2_f32_bf16 %5, %10, %13, %14\n\t"
+      "v_dot2_f32_bf16 %6, %11, %12, %14\n\tv_dot2_f32_bf16 %7, %11, %13, %14\n\ts_nop 2"
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(a[4]), "=&v"(a[5]), "=&v"(a[6]), "=&v"(a[7])
+      : "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "s"(0x00003F80u), "s"(0x3F800000u), "v"(nmn));
+}
+__device__ __forceinline__ void bf16_mul8(const uint32_t (&y)[8], const uint32_t (&b)[8], float (&o)[8]) {
+  asm("v_dot2_f32_bf16 %0, %8, %16, 0\n\tv_dot2_f32_bf16 %1, %9, %17, 0\n\t"
+      "v_dot2_f32_bf16 %2, %10, %18, 0\n\tv_dot2_f32_bf16 %3, %11, %19, 0\n\t"
+      "v_dot2_f32_bf16 %4, %12, %20, 0\n\tv_dot2_f32_bf16 %5, %13, %21, 0\n\t"
+      "v_dot2_f32_bf16 %6, %14, %22, 0\n\tv_dot2_f32_bf16 %7, %15, %23, 0\n\ts_nop 2"
+      : "=&v"(o[0]), "=&v"(o[1]), "=&v"(o[2]), "=&v"(o[3]), "=&v"(o[4]), "=&v"(o[5]), "=&v"(o[6]), "=&v"(o[7])
+      : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(y[4]), "v"(y[5]), "v"(y[6]), "v"(y[7]), "v"(b[0]), "v"(b[1]),
+        "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]));
+}
+
 template <int BITS>
-__device__ __forceinline__ void value_code_bf16_pair(float v0, float v1, const QParams& g, const uint8_t* lds,
-                                                     uint32_t& c0, uint32_t& c1) {
-  constexpr float qmax = (float)((1 << BITS) - 1);
-  float a0 = v0 - g.mn, a1 = v1 - g.mn;
-  rnd_bf16_pair(a0, a1);
-  float n0 = __builtin_amdgcn_fmed3f(a0 * g.rsc, 0.f, 1.f), n1 = __builtin_amdgcn_fmed3f(a1 * g.rsc, 0.f, 1.f);
-  rnd_bf16_pair(n0, n1);
-  const bool up0 = n0 >= g.za, up1 = n1 >= g.za;
-  float d0 = n0 - g.za, d1 = n1 - g.za;
-  rnd_bf16_pair(d0, d1);  // |rnd(x)| = rnd(|x|): the absolute value rides on the multiply's operand
-  float p0 = __builtin_amdgcn_fmed3f(__builtin_fabsf(d0) * (up0 ? g.rpe : g.rne), 0.f, 1.f);
-  float p1 = __builtin_amdgcn_fmed3f(__builtin_fabsf(d1) * (up1 ? g.rpe : g.rne), 0.f, 1.f);
-  rnd_bf16_pair(p0, p1);
-  const float y0 = bf2f(*(const uint16_t*)(lds + (__float_as_uint(p0) >> 15)));
-  const float y1 = bf2f(*(const uint16_t*)(lds + (__float_as_uint(p1) >> 15)));
-  float o0 = y0 * (up0 ? g.pb : -g.nb), o1 = y1 * (up1 ? g.pb : -g.nb);
-  rnd_bf16_pair(o0, o1);
-  // zl + off: an integer in [-1, qmax + 1], exact in bf16 (its rounding is the identity)
-  const float q0 = g.zl + rintf(o0), q1 = g.zl + rintf(o1);
-  c0 = (uint32_t)__builtin_amdgcn_fmed3f(q0, 0.f, qmax);
-  c1 = (uint32_t)__builtin_amdgcn_fmed3f(q1, 0.f, qmax);
+__device__ __forceinline__ uint64_t value_codes8_bf16(const uint32_t* w, const BfGroup& g, const uint8_t* lds) {
+  float a[8], o[8];
+  uint32_t y[8], b[8];
+  bf16_sub8(w, g.nmn, a);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float n = rnd<MZ_BF16>(__builtin_amdgcn_fmed3f(rnd<MZ_BF16>(a[i]) * g.rsc, 0.f, 1.f));
+    const bool up = n >= g.za;
+    const float d = rnd<MZ_BF16>(n - g.za);  // |rnd(x)| = rnd(|x|): the absolute value rides on the multiply's operand
+    const float p = rnd<MZ_BF16>(__builtin_amdgcn_fmed3f(__builtin_fabsf(d) * (up ? g.rpe : g.rne), 0.f, 1.f));
+    y[i] = *(const uint16_t*)(lds + (__float_as_uint(p) >> 15));
+    b[i] = up ? g.pb : g.nb;
+  }
+  bf16_mul8(y, b, o);
+  // 32-bit words of as many whole codes as fit: sum of (bits - base) << shift,
+  // the bases subtracted together (modulo 2^32)
+  constexpr int PER = BITS <= 4 ? 8 : 4;
+  uint32_t word[8 / PER];
+#pragma unroll
+  for (int k = 0; k < 8 / PER; ++k) {
+    constexpr uint32_t ones = (uint32_t)((((uint64_t)1 << (PER * BITS)) - 1) / ((1u << BITS) - 1));
+    uint32_t acc = 0u - g.base * ones;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const float t = __builtin_amdgcn_fmed3f(rnd<MZ_BF16>(o[PER * k + i]) + 12582912.f, g.lo, g.hi);
+      acc = (__float_as_uint(t) << (i * BITS)) + acc;
+      asm("" : "+v"(acc));  // one v_lshl_add_u32 each: the sum is not regrouped
+    }
+    word[k] = acc;
+  }
+  if constexpr (PER == 8) return word[0];
+  else return (uint64_t)word[0] | ((uint64_t)word[1] << (4 * BITS));
 }
 
 // value_code<MZ_F16, BITS, true, true> with the rewrites of the bf16 pair
