@@ -95,23 +95,24 @@ __device__ __forceinline__ void quantize_lane(const float (&x)[N], int part, uin
   }
 }
 
-// ------------------------------------------------------------- bf16 pairs
-// quantize_lane of bf16 values held as they were loaded, 16 dwords of two.
-// Min and max are taken two values at a time as fp16 patterns, which order as
-// the bf16 values do (sign and magnitude); a pattern fp16 reads as infinite or
-// NaN (bf16 magnitudes from 2^121, infinities, NaN) shows in the result, and
-// such groups, like every group the finite chain does not take, run
-// quantize_lane on the unpacked values.  The kernels are bound by VALU ops, so
-// the raw dwords and the dot products' free unpacking are the gain: about 17
-// ops a value instead of 22, and 4 instead of 64 for 32 values' min and max.
-// Prefill of K and V, 64 x 8 heads x 4096 tokens x 128, 4 bits: 457 -> 400 us.
-template <int BITS>
-__device__ __forceinline__ void quantize_lane_bf16(const uint32_t (&w)[16], int part, uint8_t* prow, void* mn_out,
-                                                   void* sc_out, int64_t midx, int meta_dtype, float eps,
-                                                   const uint8_t* lds, const void* table) {
-  typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-  auto h2 = [&](uint32_t u) { return __builtin_bit_cast(h2v, u); };
-  h2v lo = h2(w[0]), hi = lo;
+// ------------------------------------------------------------- 16-bit pairs
+// quantize_lane of 16-bit values held as they were loaded, 16 dwords of two.
+// Min and max are taken two values at a time as fp16 patterns.  bf16 values
+// order as their patterns read as fp16 do (sign and magnitude); a pattern fp16
+// reads as infinite or NaN (bf16 magnitudes from 2^121, infinities, NaN) shows
+// in the result, and such groups, like every group the finite chain does not
+// take, run quantize_lane on the unpacked values.  The kernels are bound by
+// VALU ops, so the raw dwords, unpacked by the ops that read them, are the
+// gain: bf16 about 17 ops a value instead of 22, fp16 19 instead of 28, and 4
+// instead of 64 for 32 values' min and max.  Prefill of K and V, 64 x 8 heads x
+// 4096 tokens x 128, 4 bits: bf16 457 -> 400 us, fp16 563 -> 425 us.
+template <int DT, int BITS>
+__device__ __forceinline__ void quantize_lane16(const uint32_t (&w)[16], int part, uint8_t* prow, void* mn_out,
+                                                void* sc_out, int64_t midx, int meta_dtype, float eps,
+                                                const uint8_t* lds, const void* table) {
+  auto h2 = [&](uint32_t u) { return __builtin_bit_cast(f16x2v, u); };
+  auto value = [](uint32_t u) { return DT == MZ_BF16 ? bf2f((uint16_t)u) : h2f((uint16_t)u); };
+  f16x2v lo = h2(w[0]), hi = lo;
 #pragma unroll
   for (int i = 1; i < 15; i += 2) {
     lo = __builtin_elementwise_minimum(__builtin_elementwise_minimum(lo, h2(w[i])), h2(w[i + 1]));
@@ -125,15 +126,15 @@ __device__ __forceinline__ void quantize_lane_bf16(const uint32_t (&w)[16], int 
   hi = __builtin_elementwise_maximum(hi, h2(__builtin_amdgcn_alignbit(hb, hb, 16)));
   lo = __builtin_elementwise_minimum(lo, h2(dpp_sel_u<DPP_QUAD_XOR1>(__builtin_bit_cast(uint32_t, lo))));
   hi = __builtin_elementwise_maximum(hi, h2(dpp_sel_u<DPP_QUAD_XOR1>(__builtin_bit_cast(uint32_t, hi))));
-  const uint32_t mnb = __builtin_bit_cast(uint32_t, lo) << 16, mxb = __builtin_bit_cast(uint32_t, hi) << 16;
-  const bool ordered = (mnb & 0x7C000000u) != 0x7C000000u && (mxb & 0x7C000000u) != 0x7C000000u;
-  const float mn = __uint_as_float(mnb), mx = __uint_as_float(mxb);
-  const QParams g = qparams<MZ_BF16, BITS>(mn, mx, eps);
-  if (ordered && qfast<MZ_BF16>(g) && __builtin_isfinite(g.sc) && g.sc > 0.f && g.pe > 0.f && g.ne > 0.f) {
-    const BfGroup bg(g, (float)((1 << BITS) - 1));
+  const uint32_t mnb = __builtin_bit_cast(uint32_t, lo), mxb = __builtin_bit_cast(uint32_t, hi);
+  const bool ordered = (mnb & 0x7C00u) != 0x7C00u && (mxb & 0x7C00u) != 0x7C00u;
+  const float mn = value(mnb), mx = value(mxb);
+  const QParams g = qparams<DT, BITS>(mn, mx, eps);
+  if (ordered && qfast<DT>(g) && __builtin_isfinite(g.sc) && g.sc > 0.f && g.pe > 0.f && g.ne > 0.f) {
+    const typename std::conditional<DT == MZ_BF16, BfGroup, HfGroup>::type cg(g, (float)((1 << BITS) - 1));
     uint8_t* dst = prow + part * 4 * BITS;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) store_codes8<BITS>(dst + c * BITS, value_codes8_bf16<BITS>(w + 4 * c, bg, lds));
+    for (int c = 0; c < 4; ++c) store_codes8<BITS>(dst + c * BITS, value_codes8<BITS>(w + 4 * c, cg, lds));
     if (part == 0) {
       store_val(mn_out, midx, mn, meta_dtype);
       store_val(sc_out, midx, g.sc, meta_dtype);
@@ -141,8 +142,8 @@ __device__ __forceinline__ void quantize_lane_bf16(const uint32_t (&w)[16], int 
   } else {
     float x[32];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) x[2 * i] = bf2f((uint16_t)w[i]), x[2 * i + 1] = bf2f((uint16_t)(w[i] >> 16));
-    quantize_lane<MZ_BF16, BITS, 32, false>(x, part, prow, mn_out, sc_out, midx, meta_dtype, eps, lds, table);
+    for (int i = 0; i < 16; ++i) x[2 * i] = value(w[i]), x[2 * i + 1] = value(w[i] >> 16);
+    quantize_lane<DT, BITS, 32, false>(x, part, prow, mn_out, sc_out, midx, meta_dtype, eps, lds, table);
   }
 }
 
@@ -161,14 +162,14 @@ __global__ __launch_bounds__(QWG) void quantize_rows_kernel(const void* __restri
   for (int64_t row = ((int64_t)blockIdx.x * (QWG / 64) + (threadIdx.x >> 6)) * N + lane / L;
        row - lane / L < nrows; row += stride) {
     if (row < nrows) {  // lanes of a group share `row`: the whole group takes this branch
-      if constexpr (VEC && DT == MZ_BF16) {
+      if constexpr (VEC && DT != MZ_F32) {
         uint32_t w[N / 2];
 #pragma unroll
         for (int c = 0; c < N / 8; ++c) {
           const uint4 u = *(const uint4*)((const uint16_t*)x + row * xs + N * part + 8 * c);
           w[4 * c] = u.x, w[4 * c + 1] = u.y, w[4 * c + 2] = u.z, w[4 * c + 3] = u.w;
         }
-        quantize_lane_bf16<BITS>(w, part, packed + row * ps, mn, sc, row * ms, meta_dtype, eps, lds, table);
+        quantize_lane16<DT, BITS>(w, part, packed + row * ps, mn, sc, row * ms, meta_dtype, eps, lds, table);
         continue;
       }
       float v[N];
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(QWG) void quantize_values_kernel(const void* __rest
     // NARROW: every offset within a slice fits 31 bits (checked on the host)
     const int64_t src = xo + (NARROW ? (int64_t)(t * (int)st + c) : (int64_t)t * st + c);
     uint8_t* prow = packed + po + (NARROW ? (int64_t)(i * QB) : (int64_t)i * QB);
-    if constexpr (VEC && DT == MZ_BF16) {
+    if constexpr (VEC && DT != MZ_F32) {
       uint32_t w[N / 2];
 #pragma unroll
       for (int e8 = 0; e8 < N / 8; ++e8) {
@@ -258,7 +259,7 @@ __global__ __launch_bounds__(QWG) void quantize_values_kernel(const void* __rest
         const uint4 u = c + 8 * e8 < D ? *(const uint4*)((const uint16_t*)x + src + 8 * e8) : make_uint4(0, 0, 0, 0);
         w[4 * e8] = u.x, w[4 * e8 + 1] = u.y, w[4 * e8 + 2] = u.z, w[4 * e8 + 3] = u.w;
       }
-      quantize_lane_bf16<BITS>(w, part, prow, mn, sc, mo + i, meta_dtype, eps, lds, table);
+      quantize_lane16<DT, BITS>(w, part, prow, mn, sc, mo + i, meta_dtype, eps, lds, table);
       continue;
     }
     float v[N];
@@ -326,7 +327,6 @@ struct KeyStage {
     else if constexpr (DT == MZ_BF16) return bf2f(*p);
     else return h2f(*p);
   }
-  static __device__ __forceinline__ float load16(uint16_t u) { return DT == MZ_BF16 ? bf2f(u) : h2f(u); }
 };
 
 // 16-bit inputs arriving as vectors are staged transposed instead: one row
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(QWG) void quantize_keys_kernel(const void* __restri
       const int c = c0 + lane / L;
       if (c < D) {  // a group's lanes share c
         uint8_t* prow = gbase + (int64_t)c * QB;
-        if constexpr (TRANS && DT == MZ_BF16) {
+        if constexpr (TRANS) {
           static_assert(N == 32, "a lane reads 16 token-pair dwords");
           const uint4* src = (const uint4*)(tileT + c * KT_PITCH + 16 * part);
           uint32_t w[16];
@@ -462,27 +462,12 @@ __global__ __launch_bounds__(QWG) void quantize_keys_kernel(const void* __restri
             const uint4 u = src[m4];
             w[4 * m4] = u.x, w[4 * m4 + 1] = u.y, w[4 * m4 + 2] = u.z, w[4 * m4 + 3] = u.w;
           }
-          quantize_lane_bf16<BITS>(w, part, prow, mn, sc, mbase + c, meta_dtype, eps, lds, table);
+          quantize_lane16<DT, BITS>(w, part, prow, mn, sc, mbase + c, meta_dtype, eps, lds, table);
           continue;
         }
         float v[N];
-        if constexpr (TRANS) {
-          static_assert(N == 32, "a lane reads 16 token-pair dwords");
-          const uint4* src = (const uint4*)(tileT + c * KT_PITCH + 16 * part);
 #pragma unroll
-          for (int m4 = 0; m4 < 4; ++m4) {
-            const uint4 u = src[m4];
-            const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              v[8 * m4 + 2 * q] = KS::load16((uint16_t)w[q]);
-              v[8 * m4 + 2 * q + 1] = KS::load16((uint16_t)(w[q] >> 16));
-            }
-          }
-        } else {
-#pragma unroll
-          for (int k = 0; k < N; ++k) v[k] = KS::load(tile + (N * part + k) * ld + c);
-        }
+        for (int k = 0; k < N; ++k) v[k] = KS::load(tile + (N * part + k) * ld + c);
         quantize_lane<DT, BITS, N>(v, part, prow, mn, sc, mbase + c, meta_dtype, eps, lds, table);
       }
     }

@@ -241,9 +241,31 @@ __device__ __forceinline__ void bf16_mul8(const uint32_t (&y)[8], const uint32_t
         "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]));
 }
 
+// 8 codes from their biased sums t (code + M - zl, clamped): 32-bit words of as
+// many whole codes as fit, each the sum of (bits - base) << shift, the bases
+// subtracted together (modulo 2^32).
 template <int BITS>
-__device__ __forceinline__ uint64_t value_codes8_bf16(const uint32_t* w, const BfGroup& g, const uint8_t* lds) {
-  float a[8], o[8];
+__device__ __forceinline__ uint64_t pack_biased8(const float (&t)[8], uint32_t base) {
+  constexpr int PER = BITS <= 4 ? 8 : 4;
+  uint32_t word[8 / PER];
+#pragma unroll
+  for (int k = 0; k < 8 / PER; ++k) {
+    constexpr uint32_t ones = (uint32_t)((((uint64_t)1 << (PER * BITS)) - 1) / ((1u << BITS) - 1));
+    uint32_t acc = 0u - base * ones;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      acc = (__float_as_uint(t[PER * k + i]) << (i * BITS)) + acc;
+      asm("" : "+v"(acc));  // one v_lshl_add_u32 each: the sum is not regrouped
+    }
+    word[k] = acc;
+  }
+  if constexpr (PER == 8) return word[0];
+  else return (uint64_t)word[0] | ((uint64_t)word[1] << (4 * BITS));
+}
+
+template <int BITS>
+__device__ __forceinline__ uint64_t value_codes8(const uint32_t* w, const BfGroup& g, const uint8_t* lds) {
+  float a[8], o[8], t[8];
   uint32_t y[8], b[8];
   bf16_sub8(w, g.nmn, a);
 #pragma unroll
@@ -256,32 +278,65 @@ __device__ __forceinline__ uint64_t value_codes8_bf16(const uint32_t* w, const B
     b[i] = up ? g.pb : g.nb;
   }
   bf16_mul8(y, b, o);
-  // 32-bit words of as many whole codes as fit: sum of (bits - base) << shift,
-  // the bases subtracted together (modulo 2^32)
-  constexpr int PER = BITS <= 4 ? 8 : 4;
-  uint32_t word[8 / PER];
 #pragma unroll
-  for (int k = 0; k < 8 / PER; ++k) {
-    constexpr uint32_t ones = (uint32_t)((((uint64_t)1 << (PER * BITS)) - 1) / ((1u << BITS) - 1));
-    uint32_t acc = 0u - g.base * ones;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const float t = __builtin_amdgcn_fmed3f(rnd<MZ_BF16>(o[PER * k + i]) + 12582912.f, g.lo, g.hi);
-      acc = (__float_as_uint(t) << (i * BITS)) + acc;
-      asm("" : "+v"(acc));  // one v_lshl_add_u32 each: the sum is not regrouped
-    }
-    word[k] = acc;
-  }
-  if constexpr (PER == 8) return word[0];
-  else return (uint64_t)word[0] | ((uint64_t)word[1] << (4 * BITS));
+  for (int i = 0; i < 8; ++i) t[i] = __builtin_amdgcn_fmed3f(rnd<MZ_BF16>(o[i]) + 12582912.f, g.lo, g.hi);
+  return pack_biased8<BITS>(t, g.base);
 }
 
-// value_code<MZ_F16, BITS, true, true> with the rewrites of the bf16 pair
-// form, which hold for fp16 as well (they use only that 1 is an fp16 value,
-// that rounding is monotone and symmetric, and that in a finite group every
-// quotient is >= +0).  Each division is a * rcp(b) plus one residual
-// correction (qdiv; b is positive and finite here), the clamp riding on the
-// correction's FMA; p's fp16 pattern addresses the ratio table directly.
+// value_code<MZ_F16, BITS, true, true> of 8 values (4 dwords) and their packed
+// codes, with the rewrites of the bf16 form, which hold for fp16 as well (they
+// use only that 1 is an fp16 value, that rounding is monotone and symmetric,
+// and that in a finite group every quotient is >= +0).  The differences v - mn
+// (two an op) and n - za are fp16 subtractions: fp32 carries 24 >= 2 * 11 + 2
+// bits, so rounding its difference to fp16 gives the same value.  Each division
+// is a * rcp(b) plus one residual correction (qdiv; b is positive and finite
+// here), the clamp riding on the correction's FMA, the fp16 operands read as
+// they are by v_fma_mix; its fp32 result is rounded before it is converted (an
+// exact tie in fp16's subnormal range needs both).  p's fp16 pattern addresses
+// the ratio table directly.
+typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
+struct HfGroup {
+  float sc, rsc, pe, ne, rpe, rne, pb, nb, lo, hi;
+  _Float16 mn, za;
+  uint32_t base;
+  __device__ __forceinline__ HfGroup(const QParams& g, float qmax)
+      : sc(g.sc), rsc(g.rsc), pe(g.pe), ne(g.ne), rpe(g.rpe), rne(g.rne), pb(g.pb), nb(-g.nb), lo(12582912.f - g.zl),
+        hi(12582912.f - g.zl + qmax), mn((_Float16)g.mn), za((_Float16)g.za), base(__float_as_uint(lo)) {}
+};
+
+template <int BITS>
+__device__ __forceinline__ uint64_t value_codes8(const uint32_t* w, const HfGroup& g, const uint8_t* lds) {
+  const f16x2v mn2 = {g.mn, g.mn};
+  _Float16 y[8];
+  float b[8], t[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const f16x2v a2 = __builtin_bit_cast(f16x2v, w[i / 2]) - mn2;
+    const float a = (float)a2[i & 1];
+    const float n0 = __builtin_fmaf(a, g.rsc, 0.f);  // a * rsc (a >= +0): one v_fma_mix
+    const _Float16 n =
+        (_Float16)__builtin_amdgcn_fmed3f(__builtin_fmaf(__builtin_fmaf(-g.sc, n0, a), g.rsc, n0), 0.f, 1.f);
+    const bool up = n >= g.za;
+    const float d = __builtin_fabsf((float)(_Float16)(n - g.za));
+    const float q = up ? g.pe : g.ne, r = up ? g.rpe : g.rne;
+    const float p0 = __builtin_fmaf(d, r, 0.f);
+    const _Float16 p =
+        (_Float16)__builtin_amdgcn_fmed3f(__builtin_fmaf(__builtin_fmaf(-q, p0, d), r, p0), 0.f, 1.f);
+    y[i] = *(const _Float16*)(lds + (uint16_t)(__builtin_bit_cast(uint16_t, p) << 1));
+    b[i] = up ? g.pb : g.nb;
+  }
+  float one = 1.f;
+  asm("" : "+s"(one));  // opaque: o * 1 + M stays one v_fma_mix
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const _Float16 o = (_Float16)((float)y[i] * b[i]);
+    t[i] = __builtin_amdgcn_fmed3f(__builtin_fmaf((float)o, one, 12582912.f), g.lo, g.hi);
+  }
+  return pack_biased8<BITS>(t, g.base);
+}
+
+// value_codes8's fp16 chain for one value, for inputs that do not arrive as
+// aligned vectors.
 template <int BITS>
 __device__ __forceinline__ uint32_t value_code_f16(float v, const QParams& g, const uint8_t* lds) {
   constexpr float qmax = (float)((1 << BITS) - 1);

@@ -1,7 +1,8 @@
-"""The bf16 quantize kernels on the magnitudes where their path changes (GPU), bit for bit against the
-oracle: values around 2^121 (from there a bf16 pattern read as fp16 is infinite and its group takes the
-general chain), scales around 2^126 (the reciprocal of a larger one is denormal), subnormals, zeros of
-both signs, and every finite magnitude in one group, at each width."""
+"""The bf16 and fp16 quantize kernels on the magnitudes where their path changes (GPU), bit for bit
+against the oracle, at each width.  bf16: values around 2^121 (from there a bf16 pattern read as fp16 is
+infinite and its group takes the general chain), scales around 2^126 (the reciprocal of a larger one is
+denormal), subnormals, zeros of both signs, every finite magnitude in one group.  fp16: subnormals (exact
+ties of the quotients there), ordinary and largest magnitudes."""
 
 import numpy as np
 import pytest
@@ -26,9 +27,22 @@ def _patterns(lo, hi, shape, seed):
                          ids=["subnormal", "tiny", "ordinary", "edge121", "edge126", "all"])
 @pytest.mark.parametrize("bits", range(1, 9))
 def test_magnitude_edges_match_oracle(bits, lo, hi):
-    from muzero_amd.kernels import loader as L
     x = _patterns(lo, hi, (1, 2, 128, 128), 10 * bits + lo)
     x[:, :, ::5] *= torch.tensor([0.0, 1.0], dtype=torch.bfloat16).repeat(64)
+    _check(x, bits)
+
+
+@pytest.mark.parametrize("step, span", [(2.0 ** -24, 20), (2.0 ** -24, 2000), (2.0 ** -10, 3000), (16.0, 2000)],
+                         ids=["subnormal", "tiny", "ordinary", "largest"])
+@pytest.mark.parametrize("bits", range(1, 9))
+def test_fp16_magnitude_edges_match_oracle(bits, step, span):
+    g = torch.Generator().manual_seed(bits)
+    x = (torch.randint(-span, span + 1, (1, 2, 128, 128), generator=g) * step).to(torch.float16)
+    _check(x, bits)
+
+
+def _check(x, bits):
+    from muzero_amd.kernels import loader as L
     b, h, t, d = x.shape
     qb, dx, meta = 8 * bits, x.to(DEV), torch.float32
     pk = torch.empty((b, h, t // 64, d, qb), dtype=torch.uint8, device=DEV)
