@@ -250,8 +250,9 @@ def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, valu
     if keys is not None and value_prefix == key_prefix:
         storage = _storage_key(layer)
         if storage is not None:
-            key = (storage, query.dtype, query.shape, query.stride(), layer.nbits, alpha_key, alpha_value, scaling,
-                   kernel_path, mask is None)
+            # (the devices too: a tensor elsewhere goes through the checks of new arguments, which refuse it)
+            key = (storage, query.device, query.dtype, query.shape, query.stride(), layer.nbits, alpha_key, alpha_value,
+                   scaling, kernel_path, None if mask is None else mask.device)
     fast = getattr(layer, "_hip_decode", None)
     if fast is not None and key is not None and fast.key == key:
         return fast.launch(query, n_groups, r, mask), fast.kernel

@@ -1,0 +1,86 @@
+"""When a decode step may re-use the arguments cached on its layer (host logic; the launches are stand-ins that
+record what reaches them, and the tensors are on the CPU)."""
+
+import pytest
+import torch
+
+from muzero_amd import MuZeroConfig, mu_zero_decode_attention_forward
+from muzero_amd.cache import attention as A
+from muzero_amd.cache.layer import MuZeroCacheLayer
+
+B, HKV, N_REP, D, TOKENS = 2, 2, 2, 64, 5
+
+
+class _Module:
+    num_key_value_groups = N_REP
+
+
+class _Refused(Exception):
+    """A new plan's own checks refused the call."""
+
+
+class _Plan:
+    """In DecodePlan's place: refuses tensors on another device, as DecodePlan does."""
+
+    kernel = "general"
+
+    def __init__(self, query, *, attention_mask=None, k_res=None, **_):
+        for t in (query, attention_mask):
+            if t is not None and t.device != k_res.device:
+                raise _Refused
+        self.launches = ["plan"]
+
+    def run(self):
+        return self.launches
+
+
+class _Step:
+    """In StepDecode's place."""
+
+    kernel = "general"
+
+    def __init__(self, plan, key):
+        self.key, self.launches = key, plan.launches
+
+    def launch(self, query, n_groups, n_residual, mask=None):
+        self.launches.append("step")
+        return self.launches
+
+
+@pytest.fixture
+def layer(monkeypatch):
+    monkeypatch.setattr(A._k, "DecodePlan", _Plan)
+    monkeypatch.setattr(A._k, "StepDecode", _Step)
+    layer = MuZeroCacheLayer(MuZeroConfig(bits=4, residual_length=128))
+    k, v = torch.randn(2, B, HKV, TOKENS, D).bfloat16()
+    layer.update(k[:, :, :-1], v[:, :, :-1])
+    layer.update(k[:, :, -1:], v[:, :, -1:], {"materialize_full_kv": False})
+    return layer
+
+
+def _call(layer, mask=None, device="cpu"):
+    query = torch.zeros(B, HKV * N_REP, 1, D, dtype=torch.bfloat16, device=device)
+    return mu_zero_decode_attention_forward(_Module(), query, mask, 0.125, layer.get_attention_state())[0]
+
+
+def _mask(device="cpu"):
+    return torch.zeros(B, 1, 1, TOKENS, dtype=torch.bfloat16, device=device)
+
+
+def test_a_second_call_takes_the_cached_arguments(layer):
+    assert list(_call(layer, _mask())) == ["plan"]
+    assert list(_call(layer, _mask())) == ["plan", "step"]
+    assert list(_call(layer)) == ["plan"]  # without a mask: other arguments
+
+
+def test_a_mask_on_another_device_is_checked(layer):
+    _call(layer, _mask())
+    with pytest.raises(_Refused):
+        _call(layer, _mask("meta"))
+    assert list(_call(layer, _mask())) == ["plan", "step"]  # the cached arguments were not touched
+
+
+def test_a_query_on_another_device_is_checked(layer):
+    _call(layer)
+    with pytest.raises(_Refused):
+        _call(layer, device="meta")
