@@ -54,6 +54,7 @@ Kernel choice, in the reference's environment-switch style (``attention.py:92``,
 from __future__ import annotations
 
 import os
+import threading
 from collections import defaultdict
 
 import torch
@@ -230,6 +231,16 @@ def _storage_key(layer):
     return store(ks), store(vs), kr.buf.data_ptr(), kr.start, vr.buf.data_ptr(), vr.start
 
 
+def _step_owner(query: torch.Tensor):
+    """What the launch arguments cached on a layer belong to besides its storage: the stream (their workspace is
+    allocated on it, and a call on another stream would overwrite records that are still being read) and the thread
+    (which patches the arguments before it launches).  None where no cached arguments may serve: host tensors, and
+    under graph capture, whose graph must own the memory that its launches write."""
+    if not query.is_cuda or torch.cuda.is_current_stream_capturing():
+        return None
+    return _k.stream_ptr(query.device), threading.get_ident()
+
+
 def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, values, alpha_key, alpha_value, scaling,
             value_prefix, kernel_path):
     """One decode call: ``(output, fused kernel or None)``.
@@ -246,12 +257,12 @@ def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, valu
                             alpha_key, alpha_value), None
     # cached only when every pointer the arguments hold is stable across steps (residual windows in their
     # decode buffers) and the two prefixes agree
-    key = None
-    if keys is not None and value_prefix == key_prefix:
+    key, owner = None, _step_owner(query)
+    if owner is not None and keys is not None and value_prefix == key_prefix:
         storage = _storage_key(layer)
         if storage is not None:
             # (the devices too: a tensor elsewhere goes through the checks of new arguments, which refuse it)
-            key = (storage, query.device, query.dtype, query.shape, query.stride(), layer.nbits, alpha_key, alpha_value,
+            key = (storage, owner, query.device, query.dtype, query.shape, query.stride(), layer.nbits, alpha_key, alpha_value,
                    scaling, kernel_path, None if mask is None else mask.device)
     fast = getattr(layer, "_hip_decode", None)
     if fast is not None and key is not None and fast.key == key:
@@ -266,5 +277,6 @@ def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, valu
     else:
         plan = _k.UnfusedPlan(query, mask=mask, **prefix)
     out = plan.run()
-    layer._hip_decode = _k.StepDecode(plan, key) if key is not None else None
+    if owner is not None:
+        layer._hip_decode = _k.StepDecode(plan, key) if key is not None else None
     return out, plan.kernel

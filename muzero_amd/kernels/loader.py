@@ -501,8 +501,9 @@ class StepDecode:
     """The validated arguments of a :class:`DecodePlan` or :class:`UnfusedPlan`, re-launched for later decode
     steps of the same cache layer: the caller guarantees (through ``key``) that every tensor the plan points
     into is the same storage with the same strides, so only the query, the mask, the prefix / residual
-    lengths, the output and the workspace size change.  A step is one ctypes call; the workspace size and the
-    kernel are asked for again only when the lengths they depend on change."""
+    lengths, the output and the workspace size change.  One thread launches it, on one stream (also in ``key``):
+    the arguments are patched in place, and the workspace is the stream's.  A step is one ctypes call; the workspace
+    size and the kernel are asked for again only when the lengths they depend on change."""
 
     __slots__ = ("key", "args", "argp", "lib", "device", "q_dtype", "out_shape", "workspace", "_keep",
                  "_keep_query", "uses_fold", "kernel", "_sized_for", "_run", "_need", "_tile", "_align")

@@ -1,6 +1,9 @@
 """When a decode step may re-use the arguments cached on its layer (host logic; the launches are stand-ins that
 record what reaches them, and the tensors are on the CPU)."""
 
+import threading
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -51,6 +54,7 @@ class _Step:
 def layer(monkeypatch):
     monkeypatch.setattr(A._k, "DecodePlan", _Plan)
     monkeypatch.setattr(A._k, "StepDecode", _Step)
+    monkeypatch.setattr(A, "_step_owner", lambda query: (0, 0))
     layer = MuZeroCacheLayer(MuZeroConfig(bits=4, residual_length=128))
     k, v = torch.randn(2, B, HKV, TOKENS, D).bfloat16()
     layer.update(k[:, :, :-1], v[:, :, :-1])
@@ -84,3 +88,34 @@ def test_a_query_on_another_device_is_checked(layer):
     _call(layer)
     with pytest.raises(_Refused):
         _call(layer, device="meta")
+
+
+def test_other_streams_and_threads_get_their_own_arguments(layer, monkeypatch):
+    """The cached arguments hold one workspace and are patched in place: another stream's launches would overwrite
+    records still being read, another thread's patches the arguments of a launch under way."""
+    for mask in (None, _mask()):
+        for owner in ((0, 0), (1, 0), (1, 1), (0, 0)):
+            monkeypatch.setattr(A, "_step_owner", lambda query, owner=owner: owner)
+            assert list(_call(layer, mask)) == ["plan"]
+            assert list(_call(layer, mask)) == ["plan", "step"]
+
+
+def test_a_captured_call_neither_takes_nor_replaces_the_cached_arguments(layer, monkeypatch):
+    """A graph must own the memory its launches write."""
+    _call(layer)
+    cached = layer._hip_decode
+    monkeypatch.setattr(A, "_step_owner", lambda query: None)
+    assert list(_call(layer)) == ["plan"]
+    assert layer._hip_decode is cached
+
+
+def test_the_owner_is_the_stream_and_the_thread(monkeypatch):
+    owner = A._step_owner
+    gpu = SimpleNamespace(is_cuda=True, device=torch.device("cuda", 1))
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(A._k, "stream_ptr", lambda device: 100 + device.index)
+    assert owner(gpu) == (101, threading.get_ident())
+    assert owner(SimpleNamespace(is_cuda=False, device=torch.device("cpu"))) is None
+    capturing[0] = True
+    assert owner(gpu) is None
