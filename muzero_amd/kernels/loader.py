@@ -503,7 +503,9 @@ class StepDecode:
     into is the same storage with the same strides, so only the query, the mask, the prefix / residual
     lengths, the output and the workspace size change.  One thread launches it, on one stream (also in ``key``):
     the arguments are patched in place, and the workspace is the stream's.  A step is one ctypes call; the workspace
-    size and the kernel are asked for again only when the lengths they depend on change."""
+    size and the kernel are asked for again only when the lengths they depend on change.  The workspace of a fused
+    kernel is kept; that of the unfused path, which holds every logit of the call, is taken from the allocator for
+    each launch, so that a model's layers do not hold one each."""
 
     __slots__ = ("key", "args", "argp", "lib", "device", "q_dtype", "out_shape", "workspace", "_keep",
                  "_keep_query", "uses_fold", "kernel", "_sized_for", "_run", "_need", "_tile", "_align")
@@ -516,11 +518,11 @@ class StepDecode:
         self.device = plan.device
         self.q_dtype = plan.out.dtype
         self.out_shape = tuple(plan.out.shape)
-        self.workspace = plan.workspace
+        fused = plan.kernel is not None
+        self.workspace = plan.workspace if fused else None
         self._keep = plan._keep  # tables, packed/residual views: kept alive with the arguments
         self.kernel = plan.kernel
         self.uses_fold = plan.kernel == "fold"
-        fused = plan.kernel is not None
         self._run = lib.muzero_decode_attention if fused else lib.muzero_decode_unfused
         self._need = (lambda argp: lib.muzero_decode_workspace_bytes(argp, None)) if fused else \
             lib.muzero_decode_unfused_workspace_bytes
@@ -532,13 +534,15 @@ class StepDecode:
         a = self.args
         need = self._need(self.argp)
         _require(need >= 0, "decode arguments rejected")
+        if self.kernel is None:
+            a.workspace_bytes = need
+            return
         if need > a.workspace_bytes:
             self.workspace = torch.empty((need + 3) // 4, dtype=torch.float32, device=self.device)
             a.workspace = self.workspace.data_ptr()
             a.workspace_bytes = need
-        if self.kernel is not None:
-            self.kernel = DECODE_KERNELS[self.lib.muzero_decode_kernel(self.argp)]
-            self.uses_fold = self.kernel == "fold"
+        self.kernel = DECODE_KERNELS[self.lib.muzero_decode_kernel(self.argp)]
+        self.uses_fold = self.kernel == "fold"
 
     def launch(self, query: torch.Tensor, n_groups: int, n_residual: int,
                mask: torch.Tensor | None = None) -> torch.Tensor:
@@ -559,6 +563,9 @@ class StepDecode:
         if sized_for != self._sized_for:
             self._size(n_groups, n_residual)
             self._sized_for = sized_for
+        if self.kernel is None:
+            workspace = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=self.device)
+            a.workspace = workspace.data_ptr()
         status = self._run(self.argp, stream_ptr(self.device))
         if status:
             check(status, "decode")

@@ -74,3 +74,19 @@ def test_derivatives_run_the_steps():
     out, _ = mz.mu_zero_decode_attention_forward(_Module(2), q, None, 0.1, layer.get_attention_state())
     out.sum().backward()
     assert q.grad is not None and torch.isfinite(q.grad).all()
+
+
+def test_a_layer_holds_no_workspace_between_calls():
+    """The workspace holds all logits of a call: only the output may stay allocated after one, on the call that
+    builds the layer's arguments and on those that re-use them."""
+    layer = MuZeroCacheLayer(mz.MuZeroConfig(bits=4, residual_length=128))
+    k, v = torch.randn(2, 4, 2, 6000, 96, device="cuda").to(BF)
+    layer.update(k[:, :, :-1], v[:, :, :-1])
+    layer.update(k[:, :, -1:], v[:, :, -1:], {"materialize_full_kv": False})
+    q = torch.randn(4, 8, 1, 96, device="cuda").to(BF)
+    logits = 4 * 8 * 6000 * 2
+    torch.cuda.synchronize()
+    for _ in range(3):
+        before = torch.cuda.memory_allocated()
+        out, _ = mz.mu_zero_decode_attention_forward(_Module(4), q, None, 0.1, layer.get_attention_state())
+        assert torch.cuda.memory_allocated() - before < logits // 4
