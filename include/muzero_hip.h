@@ -380,16 +380,20 @@ int muzero_decode_prefix_state(const mz_decode_args* args, const mz_prefix_state
  * the library (one per device, held until the process ends); args->workspace
  * and args->workspace_bytes are ignored.  Allocates nothing, so it serves
  * callers that cannot call hipMalloc (code under HIP graph capture, tight
- * serving loops, harnesses that forbid allocation).  Returns MZ_ESCRATCH,
- * launching nothing, when a split call's muzero_decode_workspace_bytes(args)
- * exceeds the array (a single-split call of the other kernels uses no
- * workspace); a two-pass call whose logits and records exceed it runs the
- * general kernel instead (the same dequantize-then-attend values, summed in
- * another order).  Every call on a device shares that device's array (the last call's
+ * serving loops, harnesses that forbid allocation).  A call whose
+ * muzero_decode_workspace_bytes(args) fits the array, and one that the library
+ * runs in a single split without the two-pass kernel (it uses no workspace),
+ * gives the results of muzero_decode_attention with a workspace bit for bit.
+ * Otherwise, with n_split <= 0, the library halves its own split count until
+ * the records fit, and a two-pass call (5 to 8 bits) whose logits and records
+ * do not fit after three halvings runs the general kernel (the same
+ * dequantize-then-attend values) at a split count found the same way; these
+ * calls sum in another order.  With n_split > 0 the count stands: a two-pass
+ * call that does not fit runs the general kernel with it, and MZ_ESCRATCH is
+ * returned, nothing launched, when the records still exceed the array.
+ * Every call on a device shares that device's array (the last call's
  * records stay in it; each call writes every record it reads), so calls that
- * overlap on one device, on different streams or threads, race.  Same
- * results as muzero_decode_attention with a workspace, bit for bit (except
- * for the two-pass calls above that fall back to the general kernel).
+ * overlap on one device, on different streams or threads, race.
  * The first call on a device does one-time runtime set-up there (the
  * scratch array's address, a kernel's LDS limit): a caller that captures
  * the call in a HIP graph makes one call on that device before the capture

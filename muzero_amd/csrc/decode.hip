@@ -1055,28 +1055,45 @@ static hipError_t scratch_address(void** out) {
   return hipSuccess;
 }
 
+// Reduce the call's splits (where the library chooses them) or change its
+// kernel until its records fit the scratch; the bytes it then needs, its split
+// count in *ns.  The two-pass kernel, whose logits lie in the workspace too,
+// is halved at most three times: its splits are its waves, and with about a
+// tenth of them the general kernel is as fast (8-bit, 32/8 heads, 4 sequences of
+// 12000 / 15000 / 16000 tokens, which leave it 27 / 6 / 2 of its 63 splits: 80 /
+// 289 / 1613 us, the general kernel 240 / 303 / 318; 64/8 heads, one of 16384, 64
+// of 256: 51 against 88).
+static int64_t plan_noalloc(mz_decode_args* a, int* ns) {
+  const int asked = a->n_split;
+  int64_t need = muzero_decode_workspace_bytes(a, ns);
+  const auto halve = [&] {
+    a->n_split = *ns / 2;
+    need = muzero_decode_workspace_bytes(a, ns);
+  };
+  const auto over = [&] { return need > (int64_t)MZ_DECODE_SCRATCH_BYTES; };
+  if (a->batch == 0 || !over()) return need;  // (negative: refused arguments)
+  const bool own = asked <= 0;
+  if (which_kernel(a) == K_TWOPASS) {
+    for (int i = 0; own && i < 3 && over() && *ns > 1; ++i) halve();
+    if (over()) {
+      a->kernel_path = MZ_PATH_GENERAL;
+      a->n_split = asked;
+      need = muzero_decode_workspace_bytes(a, ns);
+    }
+  }
+  while (own && over() && *ns > 1) halve();
+  return need;
+}
+
 extern "C" int muzero_decode_attention_noalloc(const mz_decode_args* a, mz_stream_t stream) {
   if (!a) return MZ_EINVAL;
   mz_decode_args b = *a;
   int ns = 0;
-  int64_t need = muzero_decode_workspace_bytes(&b, &ns);
+  const int64_t need = plan_noalloc(&b, &ns);
   if (need < 0) {
     // the status muzero_decode_attention gives for the same arguments
     const int c = check_args(a);
     return c != MZ_OK ? c : MZ_EUNSUPPORTED;  // a forced fold path the fold kernel does not take
-  }
-  // where the library's own split count does not fit the scratch, fewer splits may
-  if (a->n_split <= 0 && b.batch > 0)
-    while (need > (int64_t)MZ_DECODE_SCRATCH_BYTES && ns > 1) {
-      b.n_split = ns / 2;
-      need = muzero_decode_workspace_bytes(&b, &ns);
-    }
-  // the two-pass kernel keeps its logits in the workspace as well: a call
-  // whose logits do not fit the scratch runs the general kernel instead
-  if (need > (int64_t)MZ_DECODE_SCRATCH_BYTES && b.batch > 0 && which_kernel(&b) == K_TWOPASS) {
-    b.kernel_path = MZ_PATH_GENERAL;
-    b.n_split = a->n_split;
-    need = muzero_decode_workspace_bytes(&b, &ns);
   }
   // a single split of the other kernels writes the output directly and reads no workspace
   const bool reads_ws = ns > 1 || (b.batch > 0 && which_kernel(&b) == K_TWOPASS);

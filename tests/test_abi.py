@@ -15,6 +15,7 @@ import shutil
 import subprocess
 
 import pytest
+import torch
 
 from muzero_amd import _lib
 
@@ -102,6 +103,38 @@ def test_noalloc_rejects_partials_beyond_the_scratch_without_a_device():
     assert ns.value == 64 and need == 64 * 32 * 64 * 130 * 4 > _lib.MZ_DECODE_SCRATCH_BYTES
     assert lib.muzero_decode_attention_noalloc(ctypes.byref(a), None) == _lib.MZ_ESCRATCH
     assert b"scratch" in lib.muzero_strerror(_lib.MZ_ESCRATCH)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="an accepted call would launch on its placeholder pointers")
+@pytest.mark.parametrize("batch,kv_heads,n_rep,tokens", [(129, 8, 8, 2000), (132, 8, 8, 2048), (257, 8, 4, 4096),
+                                                         (160, 8, 8, 4096), (224, 8, 8, 8192), (300, 4, 7, 4096)])
+def test_noalloc_takes_calls_whose_general_kernel_needs_fewer_splits(batch, kv_heads, n_rep, tokens):
+    """8-bit calls whose two-pass logits exceed the scratch run the general kernel. Its records at the library's
+    own split count exceed it too, so the count is reduced, to one here, which needs no records: the call passes
+    every host check and fails only for the want of a device."""
+    lib = _lib.load()
+    a = _lib.DecodeArgs()
+    a.batch, a.kv_heads, a.n_rep, a.head_dim, a.bits = batch, kv_heads, n_rep, 128, 8
+    a.n_groups, a.n_residual = tokens // 64 - 2, 128
+    a.meta_dtype, a.io_dtype, a.out_dtype = _lib.MZ_F16, _lib.MZ_BF16, _lib.MZ_BF16
+    fake = 1 << 20
+    a.query = a.k_packed = a.k_mn = a.k_scale = a.v_packed = a.v_mn = a.v_scale = fake
+    a.k_res = a.v_res = a.e_key = a.e_value = a.out = fake
+    a.q_sb, a.q_sh = kv_heads * n_rep * 128, 128
+    a.kp_sb, a.kp_sh = kv_heads * a.n_groups * 128 * 64, a.n_groups * 128 * 64
+    a.vp_sb, a.vp_sh = kv_heads * a.n_groups * 64 * 128, a.n_groups * 64 * 128
+    a.km_sb, a.km_sh, a.vm_sb, a.vm_sh = a.kp_sb // 64, a.kp_sh // 64, a.vp_sb // 64, a.vp_sh // 64
+    a.kr_sb, a.kr_sh, a.kr_st = kv_heads * 128 * 128, 128 * 128, 128
+    a.vr_sb, a.vr_sh, a.vr_st = a.kr_sb, a.kr_sh, a.kr_st
+    assert lib.muzero_decode_kernel(ctypes.byref(a)) == 3  # two-pass with a workspace
+    assert lib.muzero_decode_workspace_bytes(ctypes.byref(a), None) > _lib.MZ_DECODE_SCRATCH_BYTES
+    general = _lib.DecodeArgs.from_buffer_copy(a)
+    general.kernel_path = _lib.MZ_PATH_GENERAL
+    assert lib.muzero_decode_workspace_bytes(ctypes.byref(general), None) > _lib.MZ_DECODE_SCRATCH_BYTES
+    st = lib.muzero_decode_attention_noalloc(ctypes.byref(a), None)
+    assert st > 0, st  # a HIP error (no device), not MZ_ESCRATCH
+    a.n_split = 2  # the caller's own count stands
+    assert lib.muzero_decode_attention_noalloc(ctypes.byref(a), None) == _lib.MZ_ESCRATCH
 
 
 def test_qk_av_reject_bad_args_without_a_device():

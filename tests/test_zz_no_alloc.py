@@ -92,3 +92,36 @@ def test_noalloc_takes_fewer_splits_where_the_librarys_count_does_not_fit(hkv, n
     st, got = _noalloc(plan)
     assert st == 0
     assert (got.float() - want).abs().max().item() < 8e-3  # bf16 outputs below 1: at most an ulp apart
+
+
+def _random_args(B, hkv, n_rep, length, bits):
+    g = torch.Generator(device="cuda").manual_seed(B + length)
+    lq, d, qb = length // 64 * 64 - 64, 128, 8 * bits
+    q = torch.randn(B, hkv * n_rep, 1, d, generator=g, device="cuda").bfloat16()
+
+    def pack(shape):
+        meta = [torch.rand(*shape, 1, generator=g, device="cuda").half() for _ in range(2)]
+        return (torch.randint(0, 256, (*shape, qb), generator=g, device="cuda", dtype=torch.uint8), -meta[0] - 1, meta[1] + 2)
+    (kp, km, ks), (vp, vm, vs) = pack((B, hkv, lq // 64, d)), pack((B, hkv, lq, 2))
+    res = torch.randn(2, B, hkv, 64, d, generator=g, device="cuda").bfloat16()
+    return q, dict(bits=bits, n_groups=lq // 64, k_packed=kp, k_mn=km, k_scale=ks, v_packed=vp, v_mn=vm, v_scale=vs,
+                   k_res=res[0], v_res=res[1], alpha_key=2.0, alpha_value=2.0, scaling=d ** -0.5)
+
+
+@pytest.mark.parametrize("B,hkv,n_rep,length,kernel_path,n_split",
+                         [(129, 8, 8, 2000, "general", 1), (257, 8, 4, 1000, "general", 1),  # one split needs no records
+                          (4, 8, 4, 16000, "general", 0),   # the logits leave the two-pass kernel too few splits
+                          (4, 8, 4, 12000, "auto", 31),     # two-pass with half of its 63 splits
+                          (4, 8, 4, 15000, "auto", 6),      # with an eighth of its 59
+                          (1, 8, 8, 16384, "auto", 64)])    # and with a quarter of its 256
+def test_noalloc_reduces_splits_and_falls_back(B, hkv, n_rep, length, kernel_path, n_split):
+    """8-bit calls beyond the scratch: the kernel and the split count they run with, bit for bit."""
+    from muzero_amd.kernels import loader as L
+    q, kw = _random_args(B, hkv, n_rep, length, 8)
+    plan = L.DecodePlan(q, **kw)
+    assert plan.kernel == "twopass" and plan.args.workspace_bytes > 8 << 20
+    want = L.DecodePlan(q, kernel_path=kernel_path, n_split=n_split, **kw)
+    assert want.kernel == ("general" if kernel_path == "general" else "twopass")
+    st, got = _noalloc(plan)
+    assert st == 0, st
+    assert torch.equal(got.view(torch.int16), want.run().view(torch.int16))
