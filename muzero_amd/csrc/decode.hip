@@ -643,42 +643,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// Merge the splits of one (batch, q-head): out = sum_s e^{m_s-M} acc_s / sum_s e^{m_s-M} l_s.
+// Merge the records of one (batch, q-head): num = sum_s e^{m_s-M} acc_s, den =
+// sum_s e^{m_s-M} l_s, M the largest m_s; the result is wave 0's (a lane holds
+// D / 64 channels).  LIVE: a record without weight (l <= 0: every logit masked)
+// is left out, of M as well.
 // Bound by the latency of its loads, so they are all issued before any is
 // waited for: lane s of each wave takes record s's (m, l), and a wave sums the
 // accumulators of records wave, wave + WAVES, ... in runs of COMBINE_LOADS
-// loads (a lane holds D / 64 channels); the waves' sums meet in LDS.  One wave
-// up to 8 splits, four above.  (A loop over the splits that waits for each
-// record cost 0.5 us a split: one sequence of 1000 tokens, 4-bit, 4 / 16 splits
-// 13.2 / 19.0 us per call, now 12.7 / 12.2.)
+// loads; the waves' sums meet in LDS.  One wave up to 8 splits, four above.
+// (A loop over the splits that waits for each record cost 0.5 us a split: one
+// sequence of 1000 tokens, 4-bit, 4 / 16 splits 13.2 / 19.0 us per call, now
+// 12.7 / 12.2; the state of a prefix of 4096 tokens, 32 splits, 28.6, now 12.5.)
 constexpr int COMBINE_LOADS = 8;
-template <int D, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void decode_combine_kernel(const float* __restrict__ ws, int n_split, int Hq,
-                                                                    void* out, int out_dtype, int64_t out_sb,
-                                                                    int64_t out_sh) {
-  constexpr int C = D / 64;  // channels per lane
-  const int bh = blockIdx.x;
+template <int D, int WAVES, bool LIVE>
+__device__ __forceinline__ void merge_records(const float* __restrict__ base, int n_split, float (&num)[D / 64],
+                                              float& den, float& M_) {
+  constexpr int C = D / 64;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const float* base = ws + (int64_t)bh * n_split * (D + 2);
-  float num[C], den = 0.f, M_ = -INFINITY;
 #pragma unroll
   for (int k = 0; k < C; ++k) num[k] = 0.f;
-  // (m, l) of records 64c + lane; past 64 splits the maximum is taken first
-  float m = -INFINITY, l = 0.f;
-  if (lane < n_split) m = base[(int64_t)lane * (D + 2) + D], l = base[(int64_t)lane * (D + 2) + D + 1];
+  den = 0.f;
+  // (m, l) of record s; none past the last
+  float m, l;
+  const auto load = [&](int s) __attribute__((always_inline)) {
+    m = -INFINITY, l = 0.f;
+    if (s < n_split) m = base[(int64_t)s * (D + 2) + D], l = base[(int64_t)s * (D + 2) + D + 1];
+    if (LIVE && !(l > 0.f)) m = -INFINITY, l = 0.f;
+  };
+  // records 0..63; past 64 splits the maximum is taken first
+  load(lane);
+  const float m0 = m, l0 = l;
   float top = m;
-  for (int s = 64 + lane; s < n_split; s += 64) top = fmaxf(top, base[(int64_t)s * (D + 2) + D]);
+  for (int s = 64 + lane; s < n_split; s += 64) {
+    if constexpr (LIVE) {
+      load(s);
+      top = fmaxf(top, m);
+    } else {
+      top = fmaxf(top, base[(int64_t)s * (D + 2) + D]);
+    }
+  }
   M_ = wave_max_fast(top);
   if (M_ != -INFINITY) {
     for (int s0 = 0; s0 < n_split; s0 += 64) {
-      if (s0 > 0) {
-        const bool in = s0 + lane < n_split;
-        m = in ? base[(int64_t)(s0 + lane) * (D + 2) + D] : -INFINITY;
-        l = in ? base[(int64_t)(s0 + lane) * (D + 2) + D + 1] : 0.f;
-      }
+      if (s0 > 0) load(s0 + lane);
+      else m = m0, l = l0;
       const float f = __expf(m - M_);
       den += f * l;
+      const uint64_t live = LIVE ? __ballot(l > 0.f) : ~(uint64_t)0;
       const int last = min(64, n_split - s0);
       for (int r0 = wave; r0 < last; r0 += WAVES * COMBINE_LOADS) {
         float x[COMBINE_LOADS][C];
@@ -692,7 +704,7 @@ __global__ __launch_bounds__(64 * WAVES) void decode_combine_kernel(const float*
 #pragma unroll
         for (int k = 0; k < COMBINE_LOADS; ++k) {
           const int r = r0 + k * WAVES;
-          if (r < last) {
+          if (r < last && (!LIVE || (live >> r & 1))) {
             const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), r));
 #pragma unroll
             for (int c = 0; c < C; ++c) num[c] += w * x[k][c];
@@ -713,6 +725,18 @@ __global__ __launch_bounds__(64 * WAVES) void decode_combine_kernel(const float*
 #pragma unroll
       for (int c = 0; c < C; ++c) num[c] += part[w][C * lane + c];
   }
+}
+
+// The splits of one (batch, q-head) merged into the output.
+template <int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void decode_combine_kernel(const float* __restrict__ ws, int n_split, int Hq,
+                                                                    void* out, int out_dtype, int64_t out_sb,
+                                                                    int64_t out_sh) {
+  constexpr int C = D / 64;  // channels per lane
+  const int bh = blockIdx.x, lane = threadIdx.x & 63;
+  float num[C], den, M_;
+  merge_records<D, WAVES, false>(ws + (int64_t)bh * n_split * (D + 2), n_split, num, den, M_);
+  if (threadIdx.x >= 64) return;
   const int b = bh / Hq, h = bh - b * Hq;
 #pragma unroll
   for (int c = 0; c < C; ++c)
@@ -726,40 +750,33 @@ __global__ __launch_bounds__(64 * WAVES) void decode_combine_kernel(const float*
 // when requested, the records themselves as the reference's chunk partials
 // (chunks past the split count hold the empty state acc = 0, m = -inf, l = 0,
 // as an empty reference chunk does).
-template <int D>
-__global__ __launch_bounds__(D) void prefix_state_kernel(const float* __restrict__ ws, int n_split, int Hq,
-                                                         mz_prefix_state_args st) {
-  const int bh = blockIdx.x;
-  const int c = threadIdx.x;
+template <int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void prefix_state_kernel(const float* __restrict__ ws, int n_split, int Hq,
+                                                                  mz_prefix_state_args st) {
+  constexpr int C = D / 64;
+  const int bh = blockIdx.x, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float* base = ws + (int64_t)bh * n_split * (D + 2);
-  float M_ = -INFINITY;
-  for (int s = 0; s < n_split; ++s)
-    if (base[s * (D + 2) + D + 1] > 0.f) M_ = fmaxf(M_, base[s * (D + 2) + D]);
-  float acc = 0.f, l = 0.f;
-  if (M_ != -INFINITY) {
-    for (int s = 0; s < n_split; ++s) {
-      const float ls = base[s * (D + 2) + D + 1];
-      if (!(ls > 0.f)) continue;  // an empty record (every logit masked) adds nothing
-      const float f = __expf(base[s * (D + 2) + D] - M_);
-      acc += f * base[s * (D + 2) + c];
-      l += f * ls;
+  float acc[C], l, M_;
+  merge_records<D, WAVES, true>(base, n_split, acc, l, M_);
+  if (wave == 0) {
+    const int b = bh / Hq, h = bh - b * Hq;
+#pragma unroll
+    for (int c = 0; c < C; ++c) st.acc[b * st.acc_sb + (int64_t)h * st.acc_sh + C * lane + c] = acc[c];
+    if (lane == 0) {
+      st.m[b * st.ml_sb + h] = M_;
+      st.l[b * st.ml_sb + h] = l;
     }
   }
-  const int b = bh / Hq, h = bh - b * Hq;
-  st.acc[b * st.acc_sb + (int64_t)h * st.acc_sh + c] = acc;
-  if (c == 0) {
-    st.m[b * st.ml_sb + h] = M_;
-    st.l[b * st.ml_sb + h] = l;
-  }
-  if (st.n_chunks > 0) {
-    for (int s = 0; s < st.n_chunks; ++s) {
-      const bool real = s < n_split;
-      const int64_t row = (int64_t)bh * st.n_chunks + s;
-      st.part_acc[row * D + c] = real ? base[s * (D + 2) + c] : 0.f;
-      if (c == 0) {
-        st.part_m[row] = real ? base[s * (D + 2) + D] : -INFINITY;
-        st.part_l[row] = real ? base[s * (D + 2) + D + 1] : 0.f;
-      }
+#pragma unroll 4
+  for (int s = wave; s < st.n_chunks; s += WAVES) {
+    const bool real = s < n_split;
+    const int64_t row = (int64_t)bh * st.n_chunks + s;
+#pragma unroll
+    for (int c = C * lane; c < C * lane + C; ++c) st.part_acc[row * D + c] = real ? base[(int64_t)s * (D + 2) + c] : 0.f;
+    if (lane == 0) {
+      st.part_m[row] = real ? base[(int64_t)s * (D + 2) + D] : -INFINITY;
+      st.part_l[row] = real ? base[(int64_t)s * (D + 2) + D + 1] : 0.f;
     }
   }
 }
@@ -1007,12 +1024,9 @@ extern "C" int muzero_decode_prefix_state(const mz_decode_args* a, const mz_pref
   const int r = muzero_decode_partials(&b, stream);
   if (r != MZ_OK) return r;
   const int Hq = b.kv_heads * b.n_rep;
-  if (b.head_dim == 128)
-    hipLaunchKernelGGL((prefix_state_kernel<128>), dim3(b.batch * Hq), dim3(128), 0, s,
-                       (const float*)b.workspace, ns, Hq, *st);
-  else
-    hipLaunchKernelGGL((prefix_state_kernel<64>), dim3(b.batch * Hq), dim3(64), 0, s,
-                       (const float*)b.workspace, ns, Hq, *st);
+  const auto kernel = b.head_dim == 128 ? (ns <= 8 ? prefix_state_kernel<128, 1> : prefix_state_kernel<128, 4>)
+                                        : (ns <= 8 ? prefix_state_kernel<64, 1> : prefix_state_kernel<64, 4>);
+  hipLaunchKernelGGL(kernel, dim3(b.batch * Hq), dim3(ns <= 8 ? 64 : 256), 0, s, (const float*)b.workspace, ns, Hq, *st);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? MZ_OK : (int)e;
 }
