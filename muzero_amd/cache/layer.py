@@ -456,14 +456,15 @@ class MuZeroCacheLayer:
 
     def dense_kv(self) -> tuple[torch.Tensor, torch.Tensor]:
         """Keys and values of every cached token, ``[B, H, T, D]`` in the layer dtype: the
-        packed prefix dequantised, then the residual tail."""
+        packed prefix dequantised, then the residual tail (a tail of another dtype promotes
+        as concatenation does)."""
         return self._dense("key"), self._dense("value")
 
     def _dense(self, kind: str) -> torch.Tensor:
         store, tail = (self._kstore, self.keys) if kind == "key" else (self._vstore, self.values)
         if not store.count:
             return tail
-        if tail.dim() != 4 or has_derivatives(tail):
+        if tail.dim() != 4 or tail.dtype != self.dtype or has_derivatives(tail):
             return torch.cat([self._dequantize_span(kind, 0, store.count), tail], dim=2)
         return self._dequantize_span(kind, 0, store.count, tail)
 

@@ -90,3 +90,21 @@ def test_dense_read_keeps_the_tail_in_the_graph():
     assert torch.equal(dense.detach(), plain_layer_keys)
     dense.float().sum().backward()
     assert torch.equal(tail.grad, torch.ones_like(tail))
+
+
+@pytest.mark.parametrize("first,then", [((BF, BF), (F32, F32)), ((F16, F16), (BF, BF)), ((BF, F32), (BF, F32))])
+def test_dense_read_promotes_a_tail_of_another_dtype(first, then):
+    """A chunk in another dtype than the first, or values in another dtype than the keys: the prefix comes in the
+    layer dtype (the keys' first), and the whole is promoted with the tail as concatenation promotes it."""
+    import muzero_amd as mz
+    g = torch.Generator(device="cuda").manual_seed(4)
+    new = lambda t, dtype: torch.randn(1, 2, t, 64, generator=g, device="cuda").to(dtype)
+    layer = mz.MuZeroCacheLayer(mz.MuZeroConfig(bits=4, residual_length=128))
+    layer.update(new(512, first[0]), new(512, first[1]))
+    got = layer.update(new(7, then[0]), new(7, then[1]))
+    prefix = layer._dequantize_key_prefix(), layer._dequantize_value_prefix()
+    for dense, head, tail in zip(got, prefix, (layer.keys, layer.values)):
+        assert head.dtype == first[0] and head.shape[2] == 384 and tail.shape[2] == 135
+        want = torch.cat([head, tail], 2)
+        assert dense.dtype == want.dtype and torch.equal(dense, want)
+    assert got[1].dtype == F32
