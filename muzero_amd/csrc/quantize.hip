@@ -45,15 +45,7 @@ template <int DT, int BITS>
 __device__ __forceinline__ void quantize_chunk8(const float* x, const QParams& g, bool finite, uint8_t* dst,
                                                 const uint8_t* lds, const void* table) {
   uint64_t w = 0;
-  if (qfast<DT>(g) && finite) {
-    if constexpr (DT == MZ_F16) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) w |= (uint64_t)value_code_f16<BITS>(x[i], g, lds) << (i * BITS);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) w |= (uint64_t)value_code<DT, BITS, true, true>(x[i], g, lds, table) << (i * BITS);
-    }
-  } else if (finite) {
+  if (finite) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) w |= (uint64_t)value_code<DT, BITS, false, true>(x[i], g, lds, table) << (i * BITS);
   } else if (qfast<DT>(g)) {
@@ -70,9 +62,9 @@ __device__ __forceinline__ void quantize_chunk8(const float* x, const QParams& g
 // its group, which 64 / N lanes share) and store its N*BITS/8 packed bytes
 // at prow + part*N*BITS/8; lane part 0 stores the group's metadata at index
 // midx.  The group's parameters are formed once per lane, so a larger N
-// spreads them over more values.  FINITE = false: the caller has found the
-// group outside the finite chain.
-template <int DT, int BITS, int N, bool FINITE = true>
+// spreads them over more values.  fp32 inputs, and the 16-bit groups that
+// quantize_lane16 finds outside its finite chain.
+template <int DT, int BITS, int N>
 __device__ __forceinline__ void quantize_lane(const float (&x)[N], int part, uint8_t* prow, void* mn_out,
                                               void* sc_out, int64_t midx, int meta_dtype, float eps,
                                               const uint8_t* lds, const void* table) {
@@ -81,10 +73,9 @@ __device__ __forceinline__ void quantize_lane(const float (&x)[N], int part, uin
   const float mx = group_max<L>(tree_max<N>(x));
   QParams g = qparams<DT, BITS>(mn, mx, eps);
   if constexpr (DT == MZ_F32 && BITS >= 5) set_estimate<BITS>(g, lds, table);
-  // (fp16 rounds eps to 0: a constant group, or za at 0 or 1, then divides by 0).
   // The fp32 8-bit thresholds stay in global memory, where the plain form's
   // binary search measured faster.
-  const bool finite = FINITE && QTable<DT, BITS>::IN_LDS && __builtin_isfinite(g.mn) && __builtin_isfinite(g.sc) &&
+  const bool finite = DT == MZ_F32 && QTable<DT, BITS>::IN_LDS && __builtin_isfinite(g.mn) && __builtin_isfinite(g.sc) &&
                       g.sc > 0.f && g.pe > 0.f && g.ne > 0.f;
   uint8_t* dst = prow + part * (N / 8) * BITS;
 #pragma unroll
@@ -96,7 +87,10 @@ __device__ __forceinline__ void quantize_lane(const float (&x)[N], int part, uin
 }
 
 // ------------------------------------------------------------- 16-bit pairs
-// quantize_lane of 16-bit values held as they were loaded, 16 dwords of two.
+// quantize_lane of 16-bit values held as they were loaded, 16 dwords of two
+// (rows that cannot be read as vectors are read value by value and paired: K and
+// V of 16 x 8 heads x 4096 tokens x 100, bf16, 4 bits, 200 us by the general chain,
+// 166 paired).
 // Min and max are taken two values at a time as fp16 patterns.  bf16 values
 // order as their patterns read as fp16 do (sign and magnitude); a pattern fp16
 // reads as infinite or NaN (bf16 magnitudes from 2^121, infinities, NaN) shows
@@ -105,7 +99,9 @@ __device__ __forceinline__ void quantize_lane(const float (&x)[N], int part, uin
 // VALU ops, so the raw dwords, unpacked by the ops that read them, are the
 // gain: bf16 about 17 ops a value instead of 22, fp16 19 instead of 28, and 4
 // instead of 64 for 32 values' min and max.  Prefill of K and V, 64 x 8 heads x
-// 4096 tokens x 128, 4 bits: bf16 457 -> 400 us, fp16 563 -> 425 us.
+// 4096 tokens x 128, 4 bits: bf16 457 -> 400 us, fp16 563 -> 425 us.  (fp16 rounds
+// eps to 0: a constant group, or za at 0 or 1, then divides by 0 and is not
+// finite.)
 template <int DT, int BITS>
 __device__ __forceinline__ void quantize_lane16(const uint32_t (&w)[16], int part, uint8_t* prow, void* mn_out,
                                                 void* sc_out, int64_t midx, int meta_dtype, float eps,
@@ -143,7 +139,7 @@ __device__ __forceinline__ void quantize_lane16(const uint32_t (&w)[16], int par
     float x[32];
 #pragma unroll
     for (int i = 0; i < 16; ++i) x[2 * i] = value(w[i]), x[2 * i + 1] = value(w[i] >> 16);
-    quantize_lane<DT, BITS, 32, false>(x, part, prow, mn_out, sc_out, midx, meta_dtype, eps, lds, table);
+    quantize_lane<DT, BITS, 32>(x, part, prow, mn_out, sc_out, midx, meta_dtype, eps, lds, table);
   }
 }
 
@@ -162,20 +158,26 @@ __global__ __launch_bounds__(QWG) void quantize_rows_kernel(const void* __restri
   for (int64_t row = ((int64_t)blockIdx.x * (QWG / 64) + (threadIdx.x >> 6)) * N + lane / L;
        row - lane / L < nrows; row += stride) {
     if (row < nrows) {  // lanes of a group share `row`: the whole group takes this branch
-      if constexpr (VEC && DT != MZ_F32) {
+      if constexpr (DT != MZ_F32) {
         uint32_t w[N / 2];
+        const uint16_t* xr = (const uint16_t*)x + row * xs + N * part;
+        if constexpr (VEC) {
 #pragma unroll
-        for (int c = 0; c < N / 8; ++c) {
-          const uint4 u = *(const uint4*)((const uint16_t*)x + row * xs + N * part + 8 * c);
-          w[4 * c] = u.x, w[4 * c + 1] = u.y, w[4 * c + 2] = u.z, w[4 * c + 3] = u.w;
+          for (int c = 0; c < N / 8; ++c) {
+            const uint4 u = *(const uint4*)(xr + 8 * c);
+            w[4 * c] = u.x, w[4 * c + 1] = u.y, w[4 * c + 2] = u.z, w[4 * c + 3] = u.w;
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < N / 2; ++k) w[k] = (uint32_t)xr[2 * k] | (uint32_t)xr[2 * k + 1] << 16;
         }
         quantize_lane16<DT, BITS>(w, part, packed + row * ps, mn, sc, row * ms, meta_dtype, eps, lds, table);
-        continue;
-      }
-      float v[N];
+      } else {
+        float v[N];
 #pragma unroll
-      for (int c = 0; c < N / 8; ++c) load8<DT, VEC>(*(float(*)[8])(v + 8 * c), x, row * xs + N * part + 8 * c);
-      quantize_lane<DT, BITS, N>(v, part, packed + row * ps, mn, sc, row * ms, meta_dtype, eps, lds, table);
+        for (int c = 0; c < N / 8; ++c) load8<DT, VEC>(*(float(*)[8])(v + 8 * c), x, row * xs + N * part + 8 * c);
+        quantize_lane<DT, BITS, N>(v, part, packed + row * ps, mn, sc, row * ms, meta_dtype, eps, lds, table);
+      }
     }
   }
 }
@@ -251,30 +253,41 @@ __global__ __launch_bounds__(QWG) void quantize_values_kernel(const void* __rest
     // NARROW: every offset within a slice fits 31 bits (checked on the host)
     const int64_t src = xo + (NARROW ? (int64_t)(t * (int)st + c) : (int64_t)t * st + c);
     uint8_t* prow = packed + po + (NARROW ? (int64_t)(i * QB) : (int64_t)i * QB);
-    if constexpr (VEC && DT != MZ_F32) {
+    if constexpr (DT != MZ_F32) {
       uint32_t w[N / 2];
+      const uint16_t* xr = (const uint16_t*)x + src;
 #pragma unroll
       for (int e8 = 0; e8 < N / 8; ++e8) {
-        // D % 8 == 0: a vector lies within D or past it (lanes past D read nothing)
-        const uint4 u = c + 8 * e8 < D ? *(const uint4*)((const uint16_t*)x + src + 8 * e8) : make_uint4(0, 0, 0, 0);
-        w[4 * e8] = u.x, w[4 * e8 + 1] = u.y, w[4 * e8 + 2] = u.z, w[4 * e8 + 3] = u.w;
+        const int c8 = c + 8 * e8;
+        if constexpr (VEC) {
+          // D % 8 == 0: a vector lies within D or past it (lanes past D read nothing)
+          const uint4 u = c8 < D ? *(const uint4*)(xr + 8 * e8) : make_uint4(0, 0, 0, 0);
+          w[4 * e8] = u.x, w[4 * e8 + 1] = u.y, w[4 * e8 + 2] = u.z, w[4 * e8 + 3] = u.w;
+        } else if (c8 + 8 <= D) {
+#pragma unroll
+          for (int k = 4 * e8; k < 4 * e8 + 4; ++k) w[k] = (uint32_t)xr[2 * k] | (uint32_t)xr[2 * k + 1] << 16;
+        } else {
+          auto at = [&](int e) { return c + e < D ? (uint32_t)xr[e] : 0u; };
+#pragma unroll
+          for (int k = 4 * e8; k < 4 * e8 + 4; ++k) w[k] = at(2 * k) | at(2 * k + 1) << 16;
+        }
       }
       quantize_lane16<DT, BITS>(w, part, prow, mn, sc, mo + i, meta_dtype, eps, lds, table);
-      continue;
-    }
-    float v[N];
+    } else {
+      float v[N];
 #pragma unroll
-    for (int e8 = 0; e8 < N / 8; ++e8) {
-      float (&v8)[8] = *(float(*)[8])(v + 8 * e8);
-      const int c8 = c + 8 * e8;
-      if (c8 + 8 <= D) {  // VEC only picks the load width; lanes past D (D % 64 != 0) read nothing
-        load8<DT, VEC>(v8, x, src + 8 * e8);
-      } else {
+      for (int e8 = 0; e8 < N / 8; ++e8) {
+        float (&v8)[8] = *(float(*)[8])(v + 8 * e8);
+        const int c8 = c + 8 * e8;
+        if (c8 + 8 <= D) {  // VEC only picks the load width; lanes past D (D % 64 != 0) read nothing
+          load8<DT, VEC>(v8, x, src + 8 * e8);
+        } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v8[e] = c8 + e < D ? load_val<DT>(x, src + 8 * e8 + e) : 0.f;
+          for (int e = 0; e < 8; ++e) v8[e] = c8 + e < D ? load_val<DT>(x, src + 8 * e8 + e) : 0.f;
+        }
       }
+      quantize_lane<DT, BITS, N>(v, part, prow, mn, sc, mo + i, meta_dtype, eps, lds, table);
     }
-    quantize_lane<DT, BITS, N>(v, part, prow, mn, sc, mo + i, meta_dtype, eps, lds, table);
   }
 }
 
@@ -322,11 +335,6 @@ template <int DT>
 struct KeyStage {
   using T = typename std::conditional<DT == MZ_F32, float, uint16_t>::type;
   static constexpr int PAD = DT == MZ_F32 ? 1 : 2;
-  static __device__ __forceinline__ float load(const T* p) {
-    if constexpr (DT == MZ_F32) return *p;
-    else if constexpr (DT == MZ_BF16) return bf2f(*p);
-    else return h2f(*p);
-  }
 };
 
 // 16-bit inputs arriving as vectors are staged transposed instead: one row
@@ -453,22 +461,28 @@ __global__ __launch_bounds__(QWG) void quantize_keys_kernel(const void* __restri
       const int c = c0 + lane / L;
       if (c < D) {  // a group's lanes share c
         uint8_t* prow = gbase + (int64_t)c * QB;
-        if constexpr (TRANS) {
-          static_assert(N == 32, "a lane reads 16 token-pair dwords");
-          const uint4* src = (const uint4*)(tileT + c * KT_PITCH + 16 * part);
+        if constexpr (DT != MZ_F32) {
+          static_assert(N == 32, "a lane takes 16 token-pair dwords");
           uint32_t w[16];
+          if constexpr (TRANS) {
+            const uint4* src = (const uint4*)(tileT + c * KT_PITCH + 16 * part);
 #pragma unroll
-          for (int m4 = 0; m4 < 4; ++m4) {
-            const uint4 u = src[m4];
-            w[4 * m4] = u.x, w[4 * m4 + 1] = u.y, w[4 * m4 + 2] = u.z, w[4 * m4 + 3] = u.w;
+            for (int m4 = 0; m4 < 4; ++m4) {
+              const uint4 u = src[m4];
+              w[4 * m4] = u.x, w[4 * m4 + 1] = u.y, w[4 * m4 + 2] = u.z, w[4 * m4 + 3] = u.w;
+            }
+          } else {
+            const ET* col = tile + (N * part) * ld + c;
+#pragma unroll
+            for (int k = 0; k < 16; ++k) w[k] = (uint32_t)col[(2 * k) * ld] | (uint32_t)col[(2 * k + 1) * ld] << 16;
           }
           quantize_lane16<DT, BITS>(w, part, prow, mn, sc, mbase + c, meta_dtype, eps, lds, table);
-          continue;
-        }
-        float v[N];
+        } else {
+          float v[N];
 #pragma unroll
-        for (int k = 0; k < N; ++k) v[k] = KS::load(tile + (N * part + k) * ld + c);
-        quantize_lane<DT, BITS, N>(v, part, prow, mn, sc, mbase + c, meta_dtype, eps, lds, table);
+          for (int k = 0; k < N; ++k) v[k] = tile[(N * part + k) * ld + c];
+          quantize_lane<DT, BITS, N>(v, part, prow, mn, sc, mbase + c, meta_dtype, eps, lds, table);
+        }
       }
     }
   }

@@ -335,25 +335,6 @@ __device__ __forceinline__ uint64_t value_codes8(const uint32_t* w, const HfGrou
   return pack_biased8<BITS>(t, g.base);
 }
 
-// value_codes8's fp16 chain for one value, for inputs that do not arrive as
-// aligned vectors.
-template <int BITS>
-__device__ __forceinline__ uint32_t value_code_f16(float v, const QParams& g, const uint8_t* lds) {
-  constexpr float qmax = (float)((1 << BITS) - 1);
-  const float a = rnd<MZ_F16>(v - g.mn);
-  const float n0 = a * g.rsc;
-  const float n = rnd<MZ_F16>(__builtin_amdgcn_fmed3f(__builtin_fmaf(__builtin_fmaf(-g.sc, n0, a), g.rsc, n0), 0.f, 1.f));
-  const bool up = n >= g.za;
-  const float d = __builtin_fabsf(rnd<MZ_F16>(n - g.za));
-  const float b = up ? g.pe : g.ne, r = up ? g.rpe : g.rne;
-  const float p0 = d * r;
-  const uint32_t pat = f2h(__builtin_amdgcn_fmed3f(__builtin_fmaf(__builtin_fmaf(-b, p0, d), r, p0), 0.f, 1.f));
-  const float y = h2f(*(const uint16_t*)(lds + 2 * (pat & 0x7FFFu)));
-  const float o = rnd<MZ_F16>(y * (up ? g.pb : -g.nb));
-  // zl + off: an integer in [-1, qmax + 1], exact in fp16
-  return (uint32_t)__builtin_amdgcn_fmed3f(g.zl + rintf(o), 0.f, qmax);
-}
-
 // Min / max over the 8 lanes of a group (lanes 8k..8k+7), NaN-propagating:
 // IEEE 754-2019 minimum / maximum (v_minimum3_f32 / v_maximum3_f32), which
 // return NaN when either operand is NaN, as torch's amin / amax do.  (Between
