@@ -53,7 +53,8 @@ def test_version_and_strerror():
 @pytest.mark.skipif(shutil.which("gcc") is None, reason="gcc not available")
 @pytest.mark.parametrize("cls,cname", [(_lib.DecodeArgs, "mz_decode_args"), (_lib.PrologueArgs, "mz_prologue_args"),
                                        (_lib.QkArgs, "mz_qk_args"), (_lib.AvArgs, "mz_av_args"),
-                                       (_lib.PrefixStateArgs, "mz_prefix_state_args")])
+                                       (_lib.PrefixStateArgs, "mz_prefix_state_args"),
+                                       (_lib.DequantArgs, "mz_dequant_args")])
 def test_args_layout_matches_c(tmp_path, cls, cname):
     fields = [f for f, _ in cls._fields_]
     src = ['#include <stddef.h>', '#include <stdio.h>', f'#include "{HEADER}"', "int main(void) {",
