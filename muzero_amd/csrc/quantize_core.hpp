@@ -194,9 +194,14 @@ __device__ __forceinline__ uint32_t value_code(float v, const QParams& g, const 
 // The same values as the op-by-op chain, in fewer ops (every rewrite below is
 // exact for a finite group: mn and the scale finite, the divisors positive):
 //  - v - mn is one v_dot2_f32_bf16 on the dword as it was loaded: v * 1 + the
-//    other half * 0 - mn.  Its fp32 result may differ from the subtraction's in
-//    the last bit, never in the bf16 it rounds to (checked over all pairs of
-//    finite bf16 values, both halves);
+//    other half * 0 - mn (every value of the group is finite).  Its fp32 result
+//    may differ from the subtraction's in the last bit, never in the bf16 it
+//    rounds to: up to 15 binades apart, two 8-bit significands' difference has at
+//    most 24 bits, exact in both; further apart it lies within 2^-15 of the larger
+//    operand's binade, that operand is a bf16 value and half of the spacing of
+//    bf16 values around it is at least 2^-9 of the binade.  Subnormal operands
+//    are not flushed (the tests enumerate significand pairs and binades, and
+//    sample the subnormals);
 //  - each rounding to bf16 is one v_cvt_pk_bf16_f32 (rnd);
 //  - min(rnd(x), 1) = rnd(min(x, 1)) (1 is a bf16 value and rounding is
 //    monotone), and x >= 0, so the clamp rides on the multiply (med3 = the

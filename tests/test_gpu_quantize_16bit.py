@@ -55,7 +55,28 @@ def test_rows_read_value_by_value_match_oracle(dtype, lo, hi, bits, d, pitch):
     _check(x, bits, pitch)
 
 
-def _check(x, bits, pitch=None):
+def test_every_significand_pair_of_minimum_and_value():
+    """v - min for every pair of bf16 significands, 0 to 18 binades apart either way, of equal and opposite signs,
+    in both halves of a dword.  Groups of one minimum and 63 neighbouring values lie near their largest, where at
+    8 bits and an almost linear compander neighbouring bf16 quotients have different codes."""
+    value = lambda sign, exponent, frac: (sign << 15) | ((127 + exponent) << 7) | frac
+    groups = []
+    for distance in range(-18, 19):
+        for v_sign in (0, 1):
+            for a in range(128):
+                v = [value(v_sign, max(distance, 0), f) for f in range(128)]
+                for first in (0, 63, 65):  # 63 values each
+                    group = [value(1, max(-distance, 0), a)] + v[first:first + 63]
+                    shift = a + first // 63
+                    groups.append(group[shift % 64:] + group[:shift % 64])
+    u = torch.tensor(groups)
+    x = torch.where(u >= 32768, u - 65536, u).to(torch.int16).view(torch.bfloat16)
+    x = torch.cat([x, -x.flip(0)])  # positive minima too
+    assert x.shape[0] % 64 == 0
+    _check(x[None, None], 8, alpha=0.02)
+
+
+def _check(x, bits, pitch=None, alpha=2.0):
     from muzero_amd.kernels import loader as L
     b, h, t, d = x.shape
     qb, dx, meta = 8 * bits, x.to(DEV), torch.float32
@@ -64,13 +85,13 @@ def _check(x, bits, pitch=None):
     pk = torch.empty((b, h, t // 64, d, qb), dtype=torch.uint8, device=DEV)
     kmn = torch.empty((b, h, t // 64, d, 1), dtype=meta, device=DEV)
     ksc = torch.empty_like(kmn)
-    L.quantize_key_block_into(dx, bits, 2.0, 1e-8, pk, kmn, ksc)
+    L.quantize_key_block_into(dx, bits, alpha, 1e-8, pk, kmn, ksc)
     pv = torch.empty((b, h, t, -(-d // 64), qb), dtype=torch.uint8, device=DEV)
     vmn = torch.empty((b, h, t, -(-d // 64), 1), dtype=meta, device=DEV)
     vsc = torch.empty_like(vmn)
-    L.quantize_value_block_into(dx, bits, 2.0, 1e-8, pv, vmn, vsc)
-    for got, want in zip((pk, kmn, ksc, pv, vmn, vsc), ref.quantize_key_block(x, bits, 2.0, 64, amax_dtype=meta)
-                         + ref.quantize_value_block(x, bits, 2.0, 64, amax_dtype=meta)):
+    L.quantize_value_block_into(dx, bits, alpha, 1e-8, pv, vmn, vsc)
+    for got, want in zip((pk, kmn, ksc, pv, vmn, vsc), ref.quantize_key_block(x, bits, alpha, 64, amax_dtype=meta)
+                         + ref.quantize_value_block(x, bits, alpha, 64, amax_dtype=meta)):
         if got.dtype == torch.uint8:
             np.testing.assert_array_equal(got.cpu().numpy(), want.numpy())
         else:  # a NaN's sign and payload are the arithmetic unit's choice: by place
