@@ -232,13 +232,17 @@ def _storage_key(layer):
 
 
 def _step_owner(query: torch.Tensor):
-    """What the launch arguments cached on a layer belong to besides its storage: the stream (their workspace is
-    allocated on it, and a call on another stream would overwrite records that are still being read) and the thread
-    (which patches the arguments before it launches).  None where no cached arguments may serve: host tensors, and
-    under graph capture, whose graph must own the memory that its launches write."""
-    if not query.is_cuda or torch.cuda.is_current_stream_capturing():
+    """What the launch arguments cached on a layer belong to besides its storage: the device, the stream (their
+    workspace is allocated on it, and a call on another stream would overwrite records that are still being read) and
+    the thread (which patches the arguments before it launches).  None where no cached arguments may serve: host
+    tensors, and under graph capture, whose graph must own the memory that its launches write."""
+    if not query.is_cuda:
         return None
-    return _k.stream_ptr(query.device), threading.get_ident()
+    device = query.device
+    stream = _k.stream_ptr(device)
+    if stream and torch.cuda.is_current_stream_capturing():  # (the null stream cannot be captured)
+        return None
+    return device, stream, threading.get_ident()
 
 
 def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, values, alpha_key, alpha_value, scaling,
@@ -262,7 +266,7 @@ def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, valu
         storage = _storage_key(layer)
         if storage is not None:
             # (the devices too: a tensor elsewhere goes through the checks of new arguments, which refuse it)
-            key = (storage, owner, query.device, query.dtype, query.shape, query.stride(), layer.nbits, alpha_key, alpha_value,
+            key = (storage, owner, query.dtype, query.shape, query.stride(), layer.nbits, alpha_key, alpha_value,
                    scaling, kernel_path, None if mask is None else mask.device)
     fast = getattr(layer, "_hip_decode", None)
     if fast is not None and key is not None and fast.key == key:
@@ -278,5 +282,5 @@ def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, valu
         plan = _k.UnfusedPlan(query, mask=mask, **prefix)
     out = plan.run()
     if owner is not None:
-        layer._hip_decode = _k.StepDecode(plan, key) if key is not None else None
+        layer._hip_decode = _k.StepDecode(plan, key, owner[1]) if key is not None else None
     return out, plan.kernel

@@ -508,10 +508,11 @@ class StepDecode:
     each launch, so that a model's layers do not hold one each."""
 
     __slots__ = ("key", "args", "argp", "lib", "device", "q_dtype", "out_shape", "workspace", "_keep",
-                 "_keep_query", "uses_fold", "kernel", "_sized_for", "_run", "_need", "_tile", "_align")
+                 "_keep_query", "uses_fold", "kernel", "stream", "_sized_for", "_run", "_need", "_tile", "_align")
 
-    def __init__(self, plan, key):
+    def __init__(self, plan, key, stream):
         self.key = key
+        self.stream = stream
         self.args = plan.args
         self.argp = ctypes.byref(plan.args)
         self.lib = lib = plan._lib
@@ -566,7 +567,7 @@ class StepDecode:
         if self.kernel is None:
             workspace = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=self.device)
             a.workspace = workspace.data_ptr()
-        status = self._run(self.argp, stream_ptr(self.device))
+        status = self._run(self.argp, self.stream)
         if status:
             check(status, "decode")
         self._keep_query = q, mask  # alive until the next launch (the kernel reads them asynchronously)

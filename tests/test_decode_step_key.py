@@ -42,7 +42,7 @@ class _Step:
 
     kernel = "general"
 
-    def __init__(self, plan, key):
+    def __init__(self, plan, key, stream):
         self.key, self.launches = key, plan.launches
 
     def launch(self, query, n_groups, n_residual, mask=None):
@@ -54,7 +54,7 @@ class _Step:
 def layer(monkeypatch):
     monkeypatch.setattr(A._k, "DecodePlan", _Plan)
     monkeypatch.setattr(A._k, "StepDecode", _Step)
-    monkeypatch.setattr(A, "_step_owner", lambda query: (0, 0))
+    monkeypatch.setattr(A, "_step_owner", lambda query: (query.device, 0, 0))
     layer = MuZeroCacheLayer(MuZeroConfig(bits=4, residual_length=128))
     k, v = torch.randn(2, B, HKV, TOKENS, D).bfloat16()
     layer.update(k[:, :, :-1], v[:, :, :-1])
@@ -95,7 +95,7 @@ def test_other_streams_and_threads_get_their_own_arguments(layer, monkeypatch):
     records still being read, another thread's patches the arguments of a launch under way."""
     for mask in (None, _mask()):
         for owner in ((0, 0), (1, 0), (1, 1), (0, 0)):
-            monkeypatch.setattr(A, "_step_owner", lambda query, owner=owner: owner)
+            monkeypatch.setattr(A, "_step_owner", lambda query, owner=owner: (query.device, *owner))
             assert list(_call(layer, mask)) == ["plan"]
             assert list(_call(layer, mask)) == ["plan", "step"]
 
@@ -109,13 +109,14 @@ def test_a_captured_call_neither_takes_nor_replaces_the_cached_arguments(layer, 
     assert layer._hip_decode is cached
 
 
-def test_the_owner_is_the_stream_and_the_thread(monkeypatch):
-    owner = A._step_owner
+def test_the_owner_is_the_device_the_stream_and_the_thread(monkeypatch):
     gpu = SimpleNamespace(is_cuda=True, device=torch.device("cuda", 1))
-    capturing = [False]
+    stream, capturing = [100], [False]
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
-    monkeypatch.setattr(A._k, "stream_ptr", lambda device: 100 + device.index)
-    assert owner(gpu) == (101, threading.get_ident())
-    assert owner(SimpleNamespace(is_cuda=False, device=torch.device("cpu"))) is None
+    monkeypatch.setattr(A._k, "stream_ptr", lambda device: stream[0])
+    assert A._step_owner(gpu) == (gpu.device, 100, threading.get_ident())
+    assert A._step_owner(SimpleNamespace(is_cuda=False, device=torch.device("cpu"))) is None
     capturing[0] = True
-    assert owner(gpu) is None
+    assert A._step_owner(gpu) is None
+    stream[0], capturing[0] = 0, False
+    assert A._step_owner(gpu) == (gpu.device, 0, threading.get_ident())
