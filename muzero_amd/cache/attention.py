@@ -87,7 +87,8 @@ def mu_zero_decode_attention_forward(
     the model's 4-d additive (or boolean keep) mask whose last ``L`` columns
     cover the cache, or None.  Returns ``(out [B, 1, Hq, D], None)``, or None
     for a multi-token query or a missing layer (the caller then runs its own
-    attention, as with the reference).
+    attention, as with the reference).  Several streams and threads may read
+    one layer at a time; the layer keeps the launch arguments of the last.
     """
     layer = kv_cache_state.get("layer")
     if layer is None:

@@ -391,6 +391,7 @@ class MuZeroCacheLayer:
                              backend=self.backend)
 
     def _dequantize_rows(self, packed_q, mn, scale, kind: str) -> torch.Tensor:
+        """Reference helper, :meth:`_quantize_rows`'s counterpart: flat packed rows as values in the layer dtype."""
         alpha = self._alphas[kind]
         return dequantize_rows(packed_q, mn, scale, self.nbits, float(alpha), self.q_group_size, self.dtype,
                                amax_eps=self.amax_eps)

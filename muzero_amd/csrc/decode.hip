@@ -652,8 +652,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // accumulators of records wave, wave + WAVES, ... in runs of COMBINE_LOADS
 // loads; the waves' sums meet in LDS.  One wave up to 8 splits, four above.
 // (A loop over the splits that waits for each record cost 0.5 us a split: one
-// sequence of 1000 tokens, 4-bit, 4 / 16 splits 13.2 / 19.0 us per call, now
-// 12.7 / 12.2; the state of a prefix of 4096 tokens, 32 splits, 28.6, now 12.5.)
+// sequence of 1000 tokens, 4-bit, 4 / 16 splits 13.2 / 19.0 us per prebuilt call,
+// now 12.7 / 12.2; the state of a prefix of 4096 tokens, 32 splits, 28.6, now
+// 12.5.)
 constexpr int COMBINE_LOADS = 8;
 template <int D, int WAVES, bool LIVE>
 __device__ __forceinline__ void merge_records(const float* __restrict__ base, int n_split, float (&num)[D / 64],

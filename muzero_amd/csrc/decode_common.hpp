@@ -88,7 +88,7 @@ __device__ __forceinline__ void wave_max2_bound(float& x, float& y) {
 // one that is nearly empty); 0.3 where workgroups share a CU; 0.5 for the merge
 // of the splits.  The counts tried fill the CUs or the slots once, with the
 // fewest splits of the same number of rounds, besides 1 and 2.  Measured
-// (us; a count that fills the slots rounded up, two tiles per wave / this rule):
+// (us per prebuilt call; a count that fills the slots rounded up, two tiles per wave / this rule):
 // 4-bit, 1 sequence of 1000 tokens 16.3 / 12.3, of 4096 16.9 / 12.7; 48 of 2000
 // 57.2 / 48.0; 70 of 2000 90.1 / 76.1; 7-bit, 1 of 4096 18.2 / 14.5; head_dim 64,
 // 24 of 3001 32.4 / 25.9.

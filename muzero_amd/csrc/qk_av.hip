@@ -17,9 +17,9 @@
 //       logits.  A wave owns one or two key groups.
 //   av: rows = tokens of one value group (64 channels), lane = channel,
 //       coefficient = the token's attention weight.  A workgroup owns a
-//       (batch, kv-head, value group) or a split of its tokens; its 4 waves take every 4th 64-token
-//       chunk and add their sums through LDS in a fixed order (no atomics:
-//       results are deterministic).
+//       (batch, kv-head, value group) or a split of its tokens; its 4 waves
+//       take every 4th 64-token chunk and add their sums through LDS in a fixed
+//       order (no atomics: results are deterministic).
 // Per chunk, in the wave's LDS area: the rows' packed bytes (one row per lane,
 // 8-byte global loads, written at an odd dword pitch so that neither the
 // stores nor the per-row code reads meet on a bank), each row's
@@ -39,9 +39,9 @@
 // weighted sum, av over splits of the prefix's tokens, and the sum of the
 // splits.  Logits, weights and sums are rounded to the io dtype where torch's
 // steps round them.  As torch steps around the two launches it was 14 launches;
-// at B = 8, 2100 tokens, 32/8 heads of 96, 4-bit: 181 us per call, 37 us of
-// kernels now (qk 13, softmax 9, av 11, sum 4; av 43 before, 128 workgroups
-// walking 30 chunks each).
+// at B = 8, 2100 tokens, 32/8 heads of 96, 4-bit: 182 us per call, now 33.6
+// (profiled one at a time, when a kernel starts on an idle GPU: qk 12.8, softmax
+// 9.0, av 11.8, sum 3.9; av 43 before, 128 workgroups walking 30 chunks each).
 #include <algorithm>
 #include <atomic>
 

@@ -15,7 +15,8 @@
 //           DPP), 16-byte accesses where rows are aligned.
 // Minimum and scale are rounded to the metadata dtype between the two halves, as
 // storing them rounds them.  K and V of [1, 8, 896, 128] bf16, 4-bit: 92 us as
-// separate steps, 20 us here (two launches of 12 and 10 us).
+// separate steps, 20 us here (two launches; profiled one at a time 11.1 and
+// 10.3 us).
 #include "quantize_core.hpp"
 
 #include <algorithm>

@@ -19,11 +19,12 @@
 //   select16_kernel / select_kernel   take the three order statistics from the
 //       subsample, one workgroup per kind (both kinds in one launch).
 //
-// Measured at [16, 8, 1856, 128] fp16 (65536 values in the subsample): 15 us for
-// the keys, 19 us for the values (61 MB each), 10 us for both selections; with
-// the quantization the whole prefill went from 670 to 197 us.  A selection by
-// three 11-bit passes, as fp32 runs it, took 30 us for 16-bit values: 8 compares
-// and branches per value and pass, on one compute unit.
+// Measured at [16, 8, 1856, 128] fp16 (65536 values in the subsample), profiled
+// one at a time: 15 us for the keys, 18 us for the values (61 MB each), 9 us for
+// both selections; with the fp16 quantize chain the whole 8-bit prefill went from
+// 686 to 191 us.  A selection by three 11-bit passes, as fp32 runs it, took 30 us
+// for 16-bit values: 8 compares and branches per value and pass, on one compute
+// unit.
 #include "common.hpp"
 
 #include <algorithm>
