@@ -230,6 +230,10 @@ class MuZeroCacheLayer:
         # dropped whenever that storage is replaced
         self._hip_decode = None
 
+    def __getstate__(self) -> dict[str, Any]:
+        # a copy's storage lies elsewhere: its first decode step builds its own arguments
+        return {**self.__dict__, "_hip_decode": None}
+
     # ------------------------------------------------------------------
     # The full-precision tail
     # ------------------------------------------------------------------

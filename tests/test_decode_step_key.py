@@ -1,6 +1,8 @@
 """When a decode step may re-use the arguments cached on its layer (host logic; the launches are stand-ins that
 record what reaches them, and the tensors are on the CPU)."""
 
+import copy
+import ctypes
 import threading
 from types import SimpleNamespace
 
@@ -120,3 +122,15 @@ def test_the_owner_is_the_device_the_stream_and_the_thread(monkeypatch):
     assert A._step_owner(gpu) is None
     stream[0], capturing[0] = 0, False
     assert A._step_owner(gpu) == (gpu.device, 0, threading.get_ident())
+
+
+def test_a_copy_of_the_layer_builds_its_own_arguments(layer):
+    """A cache is copied to re-use a prompt, after masked decode steps as well; the launch arguments hold addresses
+    of the original's storage and cannot be copied."""
+    _call(layer, _mask())
+    layer._hip_decode.args = (ctypes.c_void_p * 1)(1)
+    other = copy.deepcopy(layer)
+    assert other._hip_decode is None and layer._hip_decode is not None
+    assert torch.equal(other.keys, layer.keys) and other.keys.data_ptr() != layer.keys.data_ptr()
+    assert list(_call(other, _mask())) == ["plan"]
+    assert list(_call(layer, _mask())) == ["plan", "step"]
