@@ -261,9 +261,10 @@ def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, valu
         return _split_steps(layer, n_rep, query, mask, scaling, key_prefix, value_prefix, keys, values,
                             alpha_key, alpha_value), None
     # cached only when every pointer the arguments hold is stable across steps (residual windows in their
-    # decode buffers) and the two prefixes agree
+    # decode buffers), and the two prefixes and the two windows agree
     key, owner = None, _step_owner(query)
-    if owner is not None and keys is not None and value_prefix == key_prefix:
+    if owner is not None and keys is not None and value_prefix == key_prefix and values is not None \
+            and values.shape[2] == r:
         storage = _storage_key(layer)
         if storage is not None:
             # (the devices too: a tensor elsewhere goes through the checks of new arguments, which refuse it)
@@ -280,7 +281,7 @@ def _launch(layer, module, fused, query, attention_mask, n_groups, r, keys, valu
     if fused:
         plan = _k.DecodePlan(query, attention_mask=mask, kernel_path=kernel_path, **prefix)
     else:
-        plan = _k.UnfusedPlan(query, mask=mask, **prefix)
+        plan = _k.UnfusedPlan(query, n_rep=n_rep, mask=mask, **prefix)
     out = plan.run()
     if owner is not None:
         layer._hip_decode = _k.StepDecode(plan, key, owner[1]) if key is not None else None

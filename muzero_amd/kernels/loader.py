@@ -809,7 +809,7 @@ class UnfusedPlan:
 
     kernel = None  # none of the fused kernels
 
-    def __init__(self, query: torch.Tensor, *, bits: int, n_groups: int, value_prefix: int,
+    def __init__(self, query: torch.Tensor, *, n_rep: int, bits: int, n_groups: int, value_prefix: int,
                  k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res,
                  alpha_key: float, alpha_value: float, scaling: float, mask: torch.Tensor | None):
         dev = _on_gpu(query, k_packed, k_mn, k_scale, v_packed, v_mn, v_scale, k_res, v_res, mask)
@@ -817,6 +817,7 @@ class UnfusedPlan:
         r = 0 if k_res is None else k_res.shape[2]
         length, qb, ng = GROUP * n_groups + r, _qbytes(bits), (d + GROUP - 1) // GROUP
         hkv = (k_res if k_res is not None else k_packed).shape[1]
+        _require(hq == hkv * n_rep, "query heads must equal kv heads * num_key_value_groups")
         a = _lib.DecodeArgs()
         if n_groups > 0:
             mn, sc = _meta4(k_mn, "K min"), _meta4(k_scale, "K scale")
@@ -842,14 +843,13 @@ class UnfusedPlan:
         _require(GROUP * n_groups <= value_prefix <= length, "value_prefix must lie between the key prefix and the cache's end")
         a.v_prefix = value_prefix if value_prefix != GROUP * n_groups else 0
         if r > 0:
-            n_v = length - value_prefix
-            _require(v_res is not None and v_res.shape[2] >= n_v, "residual K/V lengths differ")
+            _require(v_res is not None and v_res.shape[2] == length - value_prefix, "residual K/V lengths differ")
             a.k_res, a.kr_sb, a.kr_sh, a.kr_st = ptr(k_res), k_res.stride(0), k_res.stride(1), k_res.stride(2)
             a.v_res, a.vr_sb, a.vr_sh, a.vr_st = ptr(v_res), v_res.stride(0), v_res.stride(1), v_res.stride(2)
         if mask is not None:
             a.mask, a.mask_sb = ptr(mask), mask.stride(0)
         out = torch.empty((b, 1, hq, d), dtype=query.dtype, device=dev)
-        a.batch, a.kv_heads, a.n_rep, a.head_dim, a.bits = b, hkv, hq // hkv, d, int(bits)
+        a.batch, a.kv_heads, a.n_rep, a.head_dim, a.bits = b, hkv, n_rep, d, int(bits)
         a.n_groups, a.n_residual = int(n_groups), int(r)
         a.io_dtype = a.out_dtype = DTYPE_ENUM[query.dtype]
         a.scaling = float(scaling)

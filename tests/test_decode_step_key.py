@@ -29,10 +29,12 @@ class _Plan:
 
     kernel = "general"
 
-    def __init__(self, query, *, attention_mask=None, k_res=None, **_):
+    def __init__(self, query, *, attention_mask=None, k_res=None, v_res=None, **_):
         for t in (query, attention_mask):
             if t is not None and t.device != k_res.device:
                 raise _Refused
+        if v_res.shape[2] != k_res.shape[2]:
+            raise _Refused
         self.launches = ["plan"]
 
     def run(self):
@@ -90,6 +92,15 @@ def test_a_query_on_another_device_is_checked(layer):
     _call(layer)
     with pytest.raises(_Refused):
         _call(layer, device="meta")
+
+
+def test_windows_of_different_lengths_are_checked(layer):
+    _call(layer)
+    layer._vres.end -= 1
+    layer._vres._refresh()
+    layer._sync()
+    with pytest.raises(_Refused):
+        _call(layer)
 
 
 def test_other_streams_and_threads_get_their_own_arguments(layer, monkeypatch):

@@ -90,3 +90,18 @@ def test_a_layer_holds_no_workspace_between_calls():
         before = torch.cuda.memory_allocated()
         out, _ = mz.mu_zero_decode_attention_forward(_Module(4), q, None, 0.1, layer.get_attention_state())
         assert torch.cuda.memory_allocated() - before < logits // 4
+
+
+@pytest.mark.parametrize("fault", ["heads", "values"])
+def test_inconsistent_calls_are_refused(fault):
+    """Query heads that are not kv heads * num_key_value_groups (here of a layer without a residual, which alone would
+    tell), and a value residual longer than the tokens it is said to hold."""
+    layer = MuZeroCacheLayer(mz.MuZeroConfig(bits=4, residual_length=0 if fault == "heads" else 64))
+    k, v = torch.randn(2, 1, 2, 256, 96, device="cuda").to(BF)
+    layer.update(k, v)
+    state = layer.get_attention_state()
+    if fault == "values":
+        layer._set_tail(layer.keys[:, :, :60], layer.values)
+    q = torch.randn(1, 8, 1, 96, device="cuda").to(BF)
+    with pytest.raises((mz.kernels.loader.MuZeroHipError, RuntimeError)):
+        mz.mu_zero_decode_attention_forward(_Module(2 if fault == "heads" else 4), q, None, 0.1, state)
