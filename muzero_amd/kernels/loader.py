@@ -504,8 +504,11 @@ class StepDecode:
     lengths, the output and the workspace size change.  One thread launches it, on one stream (also in ``key``):
     the arguments are patched in place, and the workspace is the stream's.  A step is one ctypes call; the workspace
     size and the kernel are asked for again only when the lengths they depend on change.  The workspace of a fused
-    kernel is kept; that of the unfused path, which holds every logit of the call, is taken from the allocator for
-    each launch, so that a model's layers do not hold one each."""
+    kernel is kept; that of the unfused path, which holds every logit of the call, up to ``KEPT_WORKSPACE`` bytes (an
+    allocation costs 2 us of a small call's 20), above that it is taken from the allocator for each launch, so that a
+    model's layers do not hold one each (17 MB a layer at 8 sequences of 32k tokens, 32 heads of 96)."""
+
+    KEPT_WORKSPACE = 2 << 20
 
     __slots__ = ("key", "args", "argp", "lib", "device", "q_dtype", "out_shape", "workspace", "_keep",
                  "_keep_query", "uses_fold", "kernel", "stream", "_sized_for", "_run", "_need", "_tile", "_align")
@@ -520,7 +523,7 @@ class StepDecode:
         self.q_dtype = plan.out.dtype
         self.out_shape = tuple(plan.out.shape)
         fused = plan.kernel is not None
-        self.workspace = plan.workspace if fused else None
+        self.workspace = plan.workspace if fused or plan.args.workspace_bytes <= self.KEPT_WORKSPACE else None
         self._keep = plan._keep  # tables, packed/residual views: kept alive with the arguments
         self.kernel = plan.kernel
         self.uses_fold = plan.kernel == "fold"
@@ -535,15 +538,15 @@ class StepDecode:
         a = self.args
         need = self._need(self.argp)
         _require(need >= 0, "decode arguments rejected")
-        if self.kernel is None:
-            a.workspace_bytes = need
-            return
-        if need > a.workspace_bytes:
+        if self.kernel is None and need > self.KEPT_WORKSPACE:
+            self.workspace, a.workspace_bytes = None, need
+        elif self.workspace is None or need > a.workspace_bytes:
             self.workspace = torch.empty((need + 3) // 4, dtype=torch.float32, device=self.device)
             a.workspace = self.workspace.data_ptr()
             a.workspace_bytes = need
-        self.kernel = DECODE_KERNELS[self.lib.muzero_decode_kernel(self.argp)]
-        self.uses_fold = self.kernel == "fold"
+        if self.kernel is not None:
+            self.kernel = DECODE_KERNELS[self.lib.muzero_decode_kernel(self.argp)]
+            self.uses_fold = self.kernel == "fold"
 
     def launch(self, query: torch.Tensor, n_groups: int, n_residual: int,
                mask: torch.Tensor | None = None) -> torch.Tensor:
@@ -564,7 +567,7 @@ class StepDecode:
         if sized_for != self._sized_for:
             self._size(n_groups, n_residual)
             self._sized_for = sized_for
-        if self.kernel is None:
+        if self.workspace is None:
             workspace = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=self.device)
             a.workspace = workspace.data_ptr()
         status = self._run(self.argp, self.stream)

@@ -76,20 +76,43 @@ def test_derivatives_run_the_steps():
     assert q.grad is not None and torch.isfinite(q.grad).all()
 
 
-def test_a_layer_holds_no_workspace_between_calls():
+def test_a_layer_holds_no_large_workspace_between_calls():
     """The workspace holds all logits of a call: only the output may stay allocated after one, on the call that
     builds the layer's arguments and on those that re-use them."""
     layer = MuZeroCacheLayer(mz.MuZeroConfig(bits=4, residual_length=128))
-    k, v = torch.randn(2, 4, 2, 6000, 96, device="cuda").to(BF)
+    k, v = torch.randn(2, 4, 2, 60000, 96, device="cuda").to(BF)
     layer.update(k[:, :, :-1], v[:, :, :-1])
     layer.update(k[:, :, -1:], v[:, :, -1:], {"materialize_full_kv": False})
     q = torch.randn(4, 8, 1, 96, device="cuda").to(BF)
-    logits = 4 * 8 * 6000 * 2
+    logits = 4 * 8 * 60000 * 2
     torch.cuda.synchronize()
     for _ in range(3):
         before = torch.cuda.memory_allocated()
         out, _ = mz.mu_zero_decode_attention_forward(_Module(4), q, None, 0.1, layer.get_attention_state())
         assert torch.cuda.memory_allocated() - before < logits // 4
+
+
+def test_a_workspace_that_outgrows_what_a_layer_keeps(monkeypatch):
+    """Steps across the bound, both ways, give what new arguments give."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    new = lambda *shape: torch.randn(shape, generator=g, device="cuda").to(BF)
+    layer = MuZeroCacheLayer(mz.MuZeroConfig(bits=4, residual_length=64))
+    layer.update(new(2, 2, 300, 96), new(2, 2, 300, 96))
+    kept, bounds = [], A._k.StepDecode.KEPT_WORKSPACE
+    call = lambda q: mz.mu_zero_decode_attention_forward(_Module(4), q, None, 0.1, layer.get_attention_state())[0]
+    for step in range(40):
+        layer.update(new(2, 2, 1, 96), new(2, 2, 1, 96), {"materialize_full_kv": False})
+        q = new(2, 8, 1, 96)
+        if step == 2:  # between this step's workspace and that of one some tokens later
+            bounds = layer._hip_decode.args.workspace_bytes + 200
+        monkeypatch.setattr(A._k.StepDecode, "KEPT_WORKSPACE", bounds if step < 30 else 2 << 20)
+        got = call(q)
+        cached = layer._hip_decode
+        kept.append(cached.workspace is not None)
+        layer._hip_decode = None
+        assert torch.equal(got.view(torch.int16), call(q).view(torch.int16)), step
+        layer._hip_decode = cached
+    assert kept[3] and not kept[29] and kept[39]
 
 
 @pytest.mark.parametrize("fault", ["heads", "values"])
