@@ -39,7 +39,7 @@
 // weighted sum, av over splits of the prefix's tokens, and the sum of the
 // splits.  Logits, weights and sums are rounded to the io dtype where torch's
 // steps round them.  As torch steps around the two launches it was 14 launches;
-// at B = 8, 2100 tokens, 32/8 heads of 96, 4-bit: 182 us per call, now 33.6
+// at B = 8, 2100 tokens, 32/8 heads of 96, 4-bit: 182 us per call, now 33.2
 // (profiled one at a time, when a kernel starts on an idle GPU: qk 12.8, softmax
 // 9.0, av 11.8, sum 3.9; av 43 before, 128 workgroups walking 30 chunks each).
 #include <algorithm>
